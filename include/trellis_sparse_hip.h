@@ -182,10 +182,12 @@ typedef enum trellis_sparse_hip_dtype {
     TRELLIS_SPARSE_HIP_BF16 = 2
 } trellis_sparse_hip_dtype;
 
-/* Convolution schedule.  AUTO picks by channel counts and dtype: COMPACT where
- * it applies, else MASKED, else GENERIC; a schedule that does not apply falls
- * back the same way.  The choice never changes which pairs contribute, only
- * the order of fp32 summation. */
+/* Convolution schedule.  AUTO picks by channel counts and dtype: for F16/BF16
+ * with Ci % 64 == 0 and Co 16, 32 or a multiple of 64 an MFMA kernel over rows
+ * in the order of their neighbour masks (finite weights, features up to 2
+ * GiB), else COMPACT where it applies, else MASKED, else GENERIC; a schedule
+ * that does not apply falls back the same way.  The choice never changes which
+ * pairs contribute, only the order of fp32 summation. */
 typedef enum trellis_sparse_hip_conv_algo {
     TRELLIS_SPARSE_HIP_CONV_AUTO = 0,
     TRELLIS_SPARSE_HIP_CONV_GENERIC = 1,   /* one lane per output element, any channels and dtype */

@@ -1,0 +1,128 @@
+"""The AUTO policy's 16-bit conv (rows in mask order) where it can go wrong: the edges of its row blocks, every block
+shape (16 to 256 channels; small sets and sets that fill the GPU), repeated coordinates, more rows than one sort
+window, and weights that are not finite.
+
+Tolerance: both sides compute on the same rounded inputs, so they differ by their fp32 summation orders (some 1e-6 to
+1e-5 here; 1e-4 allowed) and by the one rounding to the storage type.  Sums on either side of a tie round to
+neighbouring values, one unit in the last place apart: of values with 8 (bf16) and 11 (fp16) significant bits that is
+at most 2^-7 and 2^-10 of the value."""
+import math
+
+import numpy as np
+import pytest
+
+import oracle_lib as orc
+import sparse_hip as sh
+import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+TOL = {sh.BF16: 2.0 ** -7 + 1e-4, sh.F16: 2.0 ** -10 + 1e-4}
+
+
+@pytest.fixture(scope="module")
+def backends():
+    bes = {dt: sh.Backend(0, dt) for dt in (sh.BF16, sh.F16)}
+    yield bes
+    for b in bes.values():
+        b.destroy()
+
+
+def err(got, exp):
+    return float(np.max(np.abs(got - exp) / np.maximum(1.0, np.maximum(np.abs(got), np.abs(exp)))))
+
+
+def weights(rng, ci, co, dtype):
+    return sh.storage_round(rng.standard_normal((co, 27, ci)) / math.sqrt(27 * ci), dtype)
+
+
+def run(be, coords, x, w, b, ci, co):
+    n = coords.shape[0]
+    rb = be.build_rulebook(coords)
+    xb, yb = be.upload(x), be.alloc(n * co)
+    be.conv(rb, xb, w, b, yb, ci, co)
+    y = be.download(yb).reshape(n, co)
+    rb.free()
+    return y
+
+
+def shell(n):
+    return np.ascontiguousarray(wl.make_coords(1)[:n])
+
+
+@pytest.mark.parametrize("n", [1, 15, 64, 65, 127, 129, 255, 257, 1000])
+@pytest.mark.parametrize("ci,co", [(64, 16), (128, 32), (64, 64), (192, 64), (64, 128), (128, 192), (256, 256),
+                                   (128, 384)])
+def test_block_edges(backends, n, ci, co):
+    dtype = sh.BF16 if n % 2 else sh.F16
+    rng = np.random.default_rng(n * 7 + ci + co)
+    coords = shell(n)
+    x = sh.storage_round(rng.standard_normal((n, ci)), dtype)
+    w, b = weights(rng, ci, co, dtype), (0.1 * rng.standard_normal(co)).astype(np.float32)
+    y = run(backends[dtype], coords, x, w, b, ci, co)
+    assert err(y, sh.storage_round(orc.Rulebook(coords).conv(x, w, b, ci, co), dtype)) <= TOL[dtype]
+
+
+# Row counts that take each block shape at 256 and 128 channels (64 x 64 up to 256 x 256), sampled rows.
+@pytest.mark.parametrize("ci,co,n", [(64, 256, 3000), (64, 256, 9000), (64, 256, 14648), (64, 512, 14648),
+                                     (64, 1024, 9000), (64, 1024, 14648), (64, 128, 3000), (128, 128, 14648)])
+def test_block_shapes(backends, ci, co, n):
+    dtype = sh.BF16
+    rng = np.random.default_rng(n + ci + co)
+    coords = shell(n)
+    coords = np.ascontiguousarray(coords[rng.permutation(n)])
+    x = sh.storage_round(rng.standard_normal((n, ci)), dtype)
+    w = weights(rng, ci, co, dtype)
+    y = run(backends[dtype], coords, x, w, None, ci, co)
+    step = 97
+    exp = orc.Rulebook(coords).conv(x, w, None, ci, co, rows=(0, n, step))
+    assert err(y[::step], sh.storage_round(exp, dtype)) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("ci,co", [(64, 64), (128, 128)])
+def test_repeated_coordinates(backends, ci, co):
+    """Every row of a repeated voxel has the last one as its centre neighbour."""
+    dtype = sh.F16
+    rng = np.random.default_rng(5)
+    coords = shell(900)
+    coords = np.ascontiguousarray(np.concatenate([coords, coords[::3], coords[::7]]))
+    n = coords.shape[0]
+    x = sh.storage_round(rng.standard_normal((n, ci)), dtype)
+    w = weights(rng, ci, co, dtype)
+    y = run(backends[dtype], coords, x, w, None, ci, co)
+    assert err(y, sh.storage_round(orc.Rulebook(coords).conv(x, w, None, ci, co), dtype)) <= TOL[dtype]
+
+
+def test_more_rows_than_a_sort_window(backends):
+    """419,340 rows (the sort takes 262,144 at a time), 64 -> 128: sampled rows in every part."""
+    dtype = sh.BF16
+    rng = np.random.default_rng(9)
+    coords = wl.make_coords(2)
+    n, ci, co = coords.shape[0], 64, 128
+    x = sh.storage_round(rng.standard_normal((n, ci), dtype=np.float32), dtype)
+    w = weights(rng, ci, co, dtype)
+    y = run(backends[dtype], coords, x, w, None, ci, co)
+    exp = orc.Rulebook(coords).conv(x, w, None, ci, co, rows=(0, n, 1009))
+    assert err(y[::1009], sh.storage_round(exp, dtype)) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("ci,co", [(64, 64), (128, 128), (192, 64)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_weights_that_are_not_finite(backends, ci, co, bad):
+    """A weight of one offset that is not finite reaches only rows with a neighbour there, as in the reference (192
+    input channels run the masked schedule, which multiplies by zero: that shape only has to give the others)."""
+    dtype = sh.BF16
+    rng = np.random.default_rng(ci)
+    coords = shell(700)
+    x = sh.storage_round(rng.standard_normal((700, ci)), dtype)
+    w = weights(rng, ci, co, dtype)
+    w[3, 2, 5] = bad
+    y = run(backends[dtype], coords, x, w, None, ci, co)
+    nbr = orc.Rulebook(coords).neighbors()
+    has = nbr[:, 2] >= 0
+    exp = sh.storage_round(orc.Rulebook(coords).conv(x, w, None, ci, co), dtype)
+    other = np.arange(co) != 3
+    assert err(y[:, other], exp[:, other]) <= TOL[dtype]
+    assert not np.isfinite(y[has, 3]).any()
+    if ci != 192:
+        assert err(y[~has, 3], exp[~has, 3]) <= TOL[dtype]

@@ -41,6 +41,13 @@ struct WeightKeyHash {
     }
 };
 
+// A device copy of host weights.  finite: no value is an infinity or a NaN in
+// the storage type (looked at for the MFMA conv packings only).
+struct Weight {
+    DevMem mem;
+    bool finite = true;
+};
+
 enum WeightLayout : int {
     kLayoutConvF32 = 1,   // fp32 [27][ci][co]
     kLayoutConvMfma = 2,  // storage type [27][ci/8][co][8]
@@ -85,7 +92,7 @@ struct Backend {
     LinearLt * lt = nullptr;
     DevMem lt_ws;
     // Weight cache.
-    std::unordered_map<WeightKey, DevMem, WeightKeyHash> weights;
+    std::unordered_map<WeightKey, Weight, WeightKeyHash> weights;
     std::vector<DevMem> transient;  // uncached weights of the current call
     // Device C2S maps (valid until destroy).
     std::vector<trellis_sparse_c2s_device_map *> maps;
@@ -392,18 +399,21 @@ trellis_status upload_bytes(Backend * be, const void * src, size_t bytes, DevMem
 
 // ---- weight / vector cache ---------------------------------------------------
 trellis_status get_weight(Backend * be, const float * host, size_t count, int layout, int ci, int co,
-                          const void ** dev_out) {
+                          const void ** dev_out, bool * finite_out = nullptr) {
     *dev_out = nullptr;
+    if (finite_out != nullptr) *finite_out = true;
     if (host == nullptr) return TRELLIS_STATUS_OK;
     const WeightKey key{host, count, layout, ci, co};
     if (be->policy.cache_weights) {
         auto it = be->weights.find(key);
         if (it != be->weights.end()) {
-            *dev_out = it->second.ptr;
+            *dev_out = it->second.mem.ptr;
+            if (finite_out != nullptr) *finite_out = it->second.finite;
             return TRELLIS_STATUS_OK;
         }
     }
     std::vector<unsigned char> staged;
+    bool finite = true;
     const int dt = be->policy.compute_dtype;
     switch (layout) {
         case kLayoutConvF32: {  // [co][27][ci] -> [27][ci][co]
@@ -421,6 +431,7 @@ trellis_status get_weight(Backend * be, const float * host, size_t count, int la
             staged.resize(elems * 2);
             uint16_t * w = (uint16_t *) staged.data();
             const int ci8 = ci / 8;
+            const uint16_t exponent = dt == kBF16 ? 0x7f80 : 0x7c00;  // all ones: infinity or NaN
             const int g = conv_stream_group(ci, co), wn = 16 * g;
             for (int o = 0; o < co; ++o) {
                 // Packed column of channel o.
@@ -435,6 +446,7 @@ trellis_status get_weight(Backend * be, const float * host, size_t count, int la
                             const _Float16 f = (_Float16) v;
                             memcpy(&h, &f, 2);
                         }
+                        if ((h & exponent) == exponent) finite = false;
                         w[((((size_t) k * ci8 + c / 8) * co + pos) * 8) + (c & 7)] = h;
                     }
             }
@@ -500,11 +512,12 @@ trellis_status get_weight(Backend * be, const float * host, size_t count, int la
     const trellis_status st = upload_bytes(be, staged.data(), staged.size(), &m);
     if (st != TRELLIS_STATUS_OK) return st;
     if (be->policy.cache_weights) {
-        be->weights[key] = m;
+        be->weights[key] = Weight{m, finite};
     } else {
         be->transient.push_back(m);
     }
     *dev_out = m.ptr;
+    if (finite_out != nullptr) *finite_out = finite;
     return TRELLIS_STATUS_OK;
 }
 
@@ -823,23 +836,65 @@ trellis_status op_add(trellis_sparse_backend * backend, const trellis_sparse_buf
 }
 
 // ---- rulebook -------------------------------------------------------------------
-trellis_status map_pass(Backend * be, trellis_sparse_rulebook * r, hipStream_t s);
-
-// The neighbour table of a rulebook built without it, written on first use.
-trellis_status rulebook_ensure_nbr(Backend * be, const trellis_sparse_rulebook * rc) {
+// The pair lists of a rulebook, built on first use by the convs that walk
+// them (and the pair and statistics downloads).
+trellis_status rulebook_ensure_lists(Backend * be, const trellis_sparse_rulebook * rc) {
     auto * r = const_cast<trellis_sparse_rulebook *>(rc);
-    if (r->nbr.ptr != nullptr) return TRELLIS_STATUS_OK;
-    const trellis_status st = dev_alloc(be, (size_t) r->n * 27 * 4, &r->nbr);
-    if (st != TRELLIS_STATUS_OK) return st;
-    stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
-    const trellis_status mst = map_pass(be, r, be->stream);
-    stage_end(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
-    return mst;
+    if (r->pair_dst.ptr != nullptr) return TRELLIS_STATUS_OK;
+    DevMem counts, off, src, dst;
+    trellis_status st = dev_alloc(be, (size_t) r->n_tiles * 27 * 4, &counts);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) r->n_tiles * 27 * 4, &off);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) r->n_tiles * kMapTile * 27 * 4, &src);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) r->n_tiles * kMapTile * 27, &dst);
+    if (st == TRELLIS_STATUS_OK) {
+        stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
+        st = hip_status(be,
+                        launch_map_lists((const int32_t *) r->rows.ptr, r->n, (int32_t *) counts.ptr,
+                                         (int32_t *) off.ptr, (int32_t *) src.ptr, (uint8_t *) dst.ptr,
+                                         (int32_t *) r->counters.ptr, be->stream),
+                        "pair lists");
+        stage_end(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
+    }
+    if (st != TRELLIS_STATUS_OK) {
+        for (DevMem * m : {&counts, &off, &src, &dst}) dev_release(be, m);
+        return st;
+    }
+    r->tile_counts = counts;
+    r->tile_off = off;
+    r->pair_src = src;
+    r->pair_dst = dst;
+    return TRELLIS_STATUS_OK;
 }
+
+// The rows' mask order, built on first use by the convs that take it.
+trellis_status rulebook_ensure_order(Backend * be, const trellis_sparse_rulebook * rc) {
+    auto * r = const_cast<trellis_sparse_rulebook *>(rc);
+    if (r->perm.ptr != nullptr) return TRELLIS_STATUS_OK;
+    const int64_t window = std::min<int64_t>((r->n + 4095) / 4096 * 4096, kOrderWindow);
+    DevMem bins, perm;
+    trellis_status st = dev_alloc(be, order_bins_bytes(r->n, window), &bins);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) r->n * 4, &perm);
+    if (st == TRELLIS_STATUS_OK) {
+        stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
+        st = hip_status(be,
+                        launch_order((const uint32_t *) r->mask.ptr, r->n, window, (int32_t *) bins.ptr,
+                                     (int32_t *) perm.ptr, be->stream),
+                        "mask order");
+        stage_end(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
+    }
+    dev_release(be, &bins);
+    if (st != TRELLIS_STATUS_OK) {
+        dev_release(be, &perm);
+        return st;
+    }
+    r->perm = perm;
+    return TRELLIS_STATUS_OK;
+}
+
 void rulebook_release(Backend * be, trellis_sparse_rulebook * r) {
     if (r == nullptr) return;
-    DevMem * mems[] = {&r->coords_mem, &r->table, &r->pool, &r->counters, &r->nbr, &r->mask,
-                       &r->tile_counts, &r->tile_off, &r->pair_src, &r->pair_dst};
+    DevMem * mems[] = {&r->coords_mem, &r->table, &r->pool, &r->counters, &r->rows, &r->mask,
+                       &r->tile_counts, &r->tile_off, &r->pair_src, &r->pair_dst, &r->perm};
     for (DevMem * m : mems) dev_release(be, m);
     delete r;
 }
@@ -850,27 +905,10 @@ int64_t next_pow2(int64_t v) {
     return p;
 }
 
-// Writes the neighbour table of a built map (a second pass of the map
-// kernel, which rewrites the pair lists with the same values).
-trellis_status map_pass(Backend * be, trellis_sparse_rulebook * r, hipStream_t s) {
-    return hip_status(be,
-                      launch_map_tiles(r->coords, r->n, (const uint64_t *) r->table.ptr,
-                                       r->table_slots, (const int32_t *) r->pool.ptr, (int32_t *) r->nbr.ptr,
-                                       (uint32_t *) r->mask.ptr, (int32_t *) r->tile_counts.ptr,
-                                       (int32_t *) r->tile_off.ptr, (int32_t *) r->pair_src.ptr,
-                                       (uint8_t *) r->pair_dst.ptr, (int32_t *) r->counters.ptr, s),
-                      "kernel map");
-}
-
-// Builds the brick hash and the kernel map for device coordinates `coords`
-// on stream s (the main stream unless given).  The [n][27] neighbour table
-// is written only when want_nbr (fp32 backends, whose conv reads it, and the
-// mesh extraction); the compacted conv reads the pair lists, and the
-// consumers of the table build it on first use (rulebook_ensure_nbr).
-trellis_status rulebook_build_device(Backend * be, const int32_t * coords, int64_t n, trellis_sparse_rulebook * r,
-                                     hipStream_t s = nullptr, bool want_nbr = false) {
-    if (s == nullptr) s = be->stream;
-    want_nbr = want_nbr || be->policy.compute_dtype == kF32;
+// Builds the brick hash and the kernel map (neighbour rows and masks) for
+// device coordinates `coords` on the backend stream.
+trellis_status rulebook_build_device(Backend * be, const int32_t * coords, int64_t n, trellis_sparse_rulebook * r) {
+    hipStream_t s = be->stream;
     r->n = n;
     r->coords = const_cast<int32_t *>(coords);
     r->table_slots = std::max<int64_t>(64, next_pow2(2 * n));
@@ -883,15 +921,10 @@ trellis_status rulebook_build_device(Backend * be, const int32_t * coords, int64
         {&r->table, slots * 16},
         {&r->pool, (size_t) (pool_empty_brick(n) + 1) * kBrickCells * 4},
         {&r->counters, kCounterInts * 4},
-        {&r->nbr, want_nbr ? (size_t) n * 27 * 4 : 0},
+        {&r->rows, (size_t) n * kMapRow * 4},
         {&r->mask, (size_t) n * 4},
-        {&r->tile_counts, (size_t) r->n_tiles * 27 * 4},
-        {&r->tile_off, (size_t) r->n_tiles * 27 * 4},
-        {&r->pair_src, (size_t) r->n_tiles * kMapTile * 27 * 4},
-        {&r->pair_dst, (size_t) r->n_tiles * kMapTile * 27},
     };
     for (const Need & q : need) {
-        if (q.bytes == 0) continue;
         const trellis_status st = dev_alloc(be, q.bytes, q.m);
         if (st != TRELLIS_STATUS_OK) return st;
     }
@@ -904,11 +937,10 @@ trellis_status rulebook_build_device(Backend * be, const int32_t * coords, int64
                                     r->table_slots, (int32_t *) r->pool.ptr, (int32_t *) r->counters.ptr, s));
     stage_end(be, TRELLIS_SPARSE_HIP_STAGE_HASH);
     stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
-    // One pass: neighbours (when wanted), per-tile counts and list starts,
-    // and each tile's pair lists in its fixed region.
-    const trellis_status mst = map_pass(be, r, s);
+    TSH_TRY(be, launch_map_rows(coords, n, (const uint64_t *) r->table.ptr, r->table_slots,
+                                (const int32_t *) r->pool.ptr, (int32_t *) r->rows.ptr, (uint32_t *) r->mask.ptr,
+                                (int32_t *) r->counters.ptr, s));
     stage_end(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
-    if (mst != TRELLIS_STATUS_OK) return mst;
     if (be->policy.reject_duplicates) {
         int32_t flags[4] = {0, 0, 0, 0};
         TSH_TRY(be, hipMemcpyAsync(flags, r->counters.ptr, sizeof(flags), hipMemcpyDeviceToHost, s));
@@ -971,20 +1003,31 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
         epi = *fused_epi;
     }
     CallScope scope(be);
+    const size_t wcount = (size_t) co * 27 * ci;
+    trellis_status st = TRELLIS_STATUS_OK;
     int algo = be->policy.conv_algo;
+    bool sorted = false;
+    const void * w = nullptr;
     if (algo == TRELLIS_SPARSE_HIP_CONV_AUTO) {
-        // The streamed compacted schedule multiplies valid pairs only; where it
-        // does not apply (Ci not 64 or a multiple of 128) the masked one, then the VALU one.
+        // The sorted schedule takes every MFMA shape with Ci % 64 == 0.  It
+        // multiplies a row without a neighbour at an offset by zeros, so
+        // weights that are not finite, whose products would be NaN where the
+        // reference skips the offset, run the compacted schedule, which
+        // multiplies valid pairs only.
         algo = TRELLIS_SPARSE_HIP_CONV_COMPACT;
+        if (conv_sorted_supported(dt, ci, co, n)) {
+            st = get_weight(be, weight, wcount, kLayoutConvMfmaGrouped, ci, co, &w, &sorted);
+            if (st != TRELLIS_STATUS_OK) return st;
+        }
     }
-    if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT && !conv_stream_supported(dt, ci, co)) {
+    if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT && !sorted && !conv_stream_supported(dt, ci, co)) {
         algo = TRELLIS_SPARSE_HIP_CONV_MASKED;
     }
     if (algo == TRELLIS_SPARSE_HIP_CONV_MASKED && !conv_mfma_supported(dt, ci, co)) {
         algo = TRELLIS_SPARSE_HIP_CONV_GENERIC;
     }
     const void * bd = nullptr;
-    trellis_status st = get_weight(be, bias, (size_t) co, kLayoutVector, 0, co, &bd);
+    st = get_weight(be, bias, (size_t) co, kLayoutVector, 0, co, &bd);
     if (st != TRELLIS_STATUS_OK) return st;
     if (epi.mode == kEpiNorm) {
         const void * g = nullptr;
@@ -995,20 +1038,25 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
         epi.gamma = (const float *) g;
         epi.beta = (const float *) b;
     }
-    const size_t wcount = (size_t) co * 27 * ci;
     hipError_t err;
     if (algo == TRELLIS_SPARSE_HIP_CONV_MASKED || algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
-        const void * w = nullptr;
-        st = get_weight(be, weight, wcount,
-                        algo == TRELLIS_SPARSE_HIP_CONV_COMPACT ? kLayoutConvMfmaGrouped : kLayoutConvMfma, ci, co,
-                        &w);
+        if (!sorted) {
+            st = get_weight(be, weight, wcount,
+                            algo == TRELLIS_SPARSE_HIP_CONV_COMPACT ? kLayoutConvMfmaGrouped : kLayoutConvMfma, ci, co,
+                            &w);
+            if (st != TRELLIS_STATUS_OK) return st;
+        }
+        if (sorted) {
+            st = rulebook_ensure_order(be, rulebook);
+        } else if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
+            st = rulebook_ensure_lists(be, rulebook);
+        }
         if (st != TRELLIS_STATUS_OK) return st;
         stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_CONV);
-        if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT && epi.mode == kEpiNone && conv_os_supported(dt, ci, co, n)) {
-            // Ci = Co = 64: the output-stationary kernel over the same lists.
-            err = launch_conv_os(dt, feats->ptr, (const int32_t *) rulebook->pair_src.ptr,
-                                 (const int32_t *) rulebook->tile_off.ptr, (const uint32_t *) rulebook->mask.ptr, w,
-                                 (const float *) bd, out->ptr, n, ci, co, be->stream);
+        if (sorted) {
+            err = launch_conv_sorted(dt, feats->ptr, (const int32_t *) rulebook->rows.ptr,
+                                     (const int32_t *) rulebook->perm.ptr, w, (const float *) bd, out->ptr, n, ci, co,
+                                     be->cus, be->stream, epi);
         } else if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
             err = launch_conv_mfma_stream(dt, feats->ptr, (const int32_t *) rulebook->pair_src.ptr,
                                           (const uint8_t *) rulebook->pair_dst.ptr,
@@ -1018,21 +1066,16 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
                                           ci, co, be->stream, epi,
                                           (const int32_t *) rulebook->counters.ptr + kLayoutStats);
         } else {
-            st = rulebook_ensure_nbr(be, rulebook);
-            if (st != TRELLIS_STATUS_OK) return st;
-            err = launch_conv_mfma_masked(dt, feats->ptr, (const int32_t *) rulebook->nbr.ptr,
+            err = launch_conv_mfma_masked(dt, feats->ptr, (const int32_t *) rulebook->rows.ptr,
                                           (const uint32_t *) rulebook->mask.ptr, w, (const float *) bd, out->ptr, n,
                                           ci, co, be->stream);
         }
         stage_end(be, TRELLIS_SPARSE_HIP_STAGE_CONV);
     } else {
-        const void * w = nullptr;
         st = get_weight(be, weight, wcount, kLayoutConvF32, ci, co, &w);
         if (st != TRELLIS_STATUS_OK) return st;
         stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_CONV);
-        st = rulebook_ensure_nbr(be, rulebook);
-        if (st != TRELLIS_STATUS_OK) return st;
-        err = launch_conv_generic(dt, feats->ptr, (const int32_t *) rulebook->nbr.ptr, (const float *) w,
+        err = launch_conv_generic(dt, feats->ptr, (const int32_t *) rulebook->rows.ptr, (const float *) w,
                                   (const float *) bd, out->ptr, n, ci, co, be->stream);
         stage_end(be, TRELLIS_SPARSE_HIP_STAGE_CONV);
     }
@@ -1656,7 +1699,7 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
         stage_end(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
         st = hip_status(be, err, "flex_dual_grid_mesh check");
     }
-    if (st == TRELLIS_STATUS_OK) st = rulebook_build_device(be, coords, n, r, nullptr, true);
+    if (st == TRELLIS_STATUS_OK) st = rulebook_build_device(be, coords, n, r);
     if (st == TRELLIS_STATUS_OK) {
         hipError_t err = hipMemcpyAsync(hf, flags.ptr, 16, hipMemcpyDeviceToHost, s);
         if (err == hipSuccess) err = hipMemcpyAsync(dup, r->counters.ptr, 8, hipMemcpyDeviceToHost, s);
@@ -1679,7 +1722,7 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
     int32_t quads = 0;
     if (st == TRELLIS_STATUS_OK) {
         stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
-        const int32_t * nbr = (const int32_t *) r->nbr.ptr;
+        const int32_t * nbr = (const int32_t *) r->rows.ptr;
         hipError_t err = launch_fdg_vertices(dt, coords, feats->ptr, n, channels, resolution, (float *) vert.ptr,
                                              (float *) wgt.ptr, s);
         if (err == hipSuccess) err = launch_fdg_count(dt, feats->ptr, nbr, n, channels, (int32_t *) counts.ptr, s);
@@ -1696,7 +1739,7 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
         if (st == TRELLIS_STATUS_OK) {
             stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
             st = hip_status(be,
-                            launch_fdg_faces(dt, feats->ptr, (const int32_t *) r->nbr.ptr, (const float *) wgt.ptr,
+                            launch_fdg_faces(dt, feats->ptr, (const int32_t *) r->rows.ptr, (const float *) wgt.ptr,
                                              (const int32_t *) first.ptr, n, channels, (int32_t *) faces.ptr, s),
                             "flex_dual_grid_mesh faces");
             stage_end(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
@@ -1757,8 +1800,8 @@ trellis_status op_trim(trellis_sparse_backend * backend, unsigned flags, size_t 
     size_t released = 0;
     if (flags & TRELLIS_SPARSE_TRIM_WEIGHTS) {
         for (auto & kv : be->weights) {
-            released += kv.second.bytes;
-            (void) hipFree(kv.second.ptr);
+            released += kv.second.mem.bytes;
+            (void) hipFree(kv.second.mem.ptr);
         }
         be->weights.clear();
     }
@@ -1827,7 +1870,7 @@ void op_destroy(trellis_sparse_backend * backend) {
     (void) hipStreamSynchronize(be->stream);
     for (auto * m : be->maps) map_release(be, m);
     be->maps.clear();
-    for (auto & kv : be->weights) dev_release(be, &kv.second);
+    for (auto & kv : be->weights) dev_release(be, &kv.second.mem);
     be->weights.clear();
     dev_release(be, &be->lt_ws);
     linear_lt_destroy(be->lt);
@@ -1972,6 +2015,8 @@ trellis_status trellis_sparse_hip_rulebook_stats(trellis_sparse_backend * backen
     if (backend == nullptr || rulebook == nullptr) return TRELLIS_STATUS_INVALID_ARGUMENT;
     Backend * be = tsh::as_backend(backend);
     tsh::select_device(be);
+    const trellis_status lst = tsh::rulebook_ensure_lists(be, rulebook);
+    if (lst != TRELLIS_STATUS_OK) return lst;
     int32_t ctr[tsh::kCounterInts];
     std::vector<int32_t> cnt((size_t) rulebook->n_tiles * 27);
     hipError_t err = hipMemcpyAsync(ctr, rulebook->counters.ptr, sizeof(ctr), hipMemcpyDeviceToHost, be->stream);
@@ -1998,10 +2043,14 @@ trellis_status trellis_sparse_hip_download_neighbors(trellis_sparse_backend * ba
     }
     Backend * be = tsh::as_backend(backend);
     tsh::select_device(be);
-    const trellis_status st = tsh::rulebook_ensure_nbr(be, rulebook);
+    tsh::DevMem nbr;
+    const trellis_status st = tsh::dev_alloc(be, (size_t) n * 27 * 4, &nbr);
     if (st != TRELLIS_STATUS_OK) return st;
-    hipError_t err = hipMemcpyAsync(nbr_out, rulebook->nbr.ptr, (size_t) n * 27 * 4, hipMemcpyDeviceToHost, be->stream);
+    hipError_t err = tsh::launch_rows_nbr((const int32_t *) rulebook->rows.ptr, n, (int32_t *) nbr.ptr, be->stream);
+    if (err == hipSuccess)
+        err = hipMemcpyAsync(nbr_out, nbr.ptr, (size_t) n * 27 * 4, hipMemcpyDeviceToHost, be->stream);
     if (err == hipSuccess) err = hipStreamSynchronize(be->stream);
+    tsh::dev_release(be, &nbr);
     return tsh::hip_status(be, err, "download_neighbors");
 }
 
@@ -2011,6 +2060,8 @@ trellis_status trellis_sparse_hip_download_pairs(trellis_sparse_backend * backen
     if (backend == nullptr || rulebook == nullptr || counts_out == nullptr) return TRELLIS_STATUS_INVALID_ARGUMENT;
     Backend * be = tsh::as_backend(backend);
     tsh::select_device(be);
+    const trellis_status lst = tsh::rulebook_ensure_lists(be, rulebook);
+    if (lst != TRELLIS_STATUS_OK) return lst;
     // Per-offset totals are the column sums of the per-(tile, offset) counts.
     const int64_t tiles = rulebook->n_tiles;
     std::vector<int32_t> off((size_t) tiles * 27), cnt((size_t) tiles * 27);

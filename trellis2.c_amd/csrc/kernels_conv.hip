@@ -3,7 +3,7 @@
 // out[i][o] = bias[o] + sum_k sum_c x[nbr[i][k]][c] * W[o][k][c]
 // (src/ops/sparse/trellis_sparse_cpu.c:324-373; weight [Co][27][Ci], :361).
 //
-// Three schedules, each deterministic:
+// Four schedules, each deterministic:
 //
 //  * generic  - VALU, any channel counts, any storage type.  For each output
 //               it follows the reference's operation order exactly: start at
@@ -11,6 +11,8 @@
 //               rounded fp32 dot product (no fused multiply-add) added to the
 //               row.  With fp32 storage the result is bit-identical to the
 //               reference CPU backend.
+//  * sorted   - kernels_conv_sorted.hip: bf16/fp16 storage, Ci % 64 == 0,
+//               finite weights; what the AUTO policy runs where it applies.
 //  * masked   - bf16/fp16 storage, Ci % 32 == 0, Co % 64 == 0.  Implicit GEMM
 //               on v_mfma_f32_16x16x32_{bf16,f16} with fp32 accumulation over
 //               the dense neighbour table.  A block owns 64 output rows x
@@ -20,11 +22,10 @@
 //               and read pre-packed weight fragments; row groups of 16 with no
 //               valid neighbour skip the offset, others multiply zeros for
 //               their missing neighbours.
-//  * os64     - bf16/fp16 storage, Ci = Co = 64 (the compact schedule's
-//               choice for that shape): output-stationary over the same pair
-//               lists, sums in registers for all 27 offsets, no tile sums.
 //  * compact  - bf16/fp16 storage, Ci = 64 or Ci % 128 == 0, Co % 64 == 0 or
-//               Co = 16 / 32 (one 16/32-channel block).  The same MFMA
+//               Co = 16 / 32 (one 16/32-channel block); the COMPACT policy,
+//               and AUTO where the weights are not all finite or the features
+//               exceed the sorted schedule's 2 GiB.  The same MFMA
 //               tiles driven by the kernel map's compacted per-tile pair
 //               lists, so the MFMA rows are valid (src, dst) pairs only; sums
 //               of a 256-row tile stay in LDS until one final store.  Blocks
@@ -70,8 +71,11 @@ __global__ void __launch_bounds__(256) k_conv_generic(const typename Store<DT>::
     const int64_t row0 = (int64_t) blockIdx.x * BM;
     const int col0 = blockIdx.y * BN;
     const int rows = (int) ((n - row0) < BM ? (n - row0) : BM);
-    // The block's neighbour rows: rows * 27 consecutive entries.
-    for (int e = t; e < BM * 27; e += 256) s_nbr[e] = e < rows * 27 ? nbr[row0 * 27 + e] : -1;
+    // The block's neighbour rows.
+    for (int e = t; e < BM * 27; e += 256) {
+        const int r = e / 27;
+        s_nbr[e] = e < rows * 27 ? nbr[(row0 + r) * kMapRow + (e - r * 27)] : -1;
+    }
     __syncthreads();
     if (t < 64) {
         // Offsets some row of the block has, in ascending order (a ballot
@@ -270,7 +274,7 @@ __global__ void __launch_bounds__(256) k_conv_mfma_masked(const typename Store<D
         bool live[2];
 #pragma unroll
         for (int m = 0; m < 2; ++m) {
-            src[m] = ((amask[m] >> k) & 1u) ? nbr[arow[m] * 27 + k] : -1;
+            src[m] = ((amask[m] >> k) & 1u) ? nbr[arow[m] * kMapRow + k] : -1;
             live[m] = __ballot(src[m] >= 0) != 0;
         }
         const typename Store<DT>::T * wk = w16 + (int64_t) k * ci8 * co * 8;
@@ -727,16 +731,6 @@ __global__ void __launch_bounds__(64 * NW) k_conv_mfma_stream(const typename Sto
 // share a CU.  A row's sums are formed in the same order in every layout, so
 // all of them give bit-identical outputs.
 // ---------------------------------------------------------------------------
-
-// Sum over the 16 lanes of a DPP row, left in every lane of the row:
-// rotations by 8, 4, 2 and 1 within the row (row_ror), each one VALU add.
-__device__ __forceinline__ float row16_sum(float v) {
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xf, 0xf, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x122, 0xf, 0xf, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false));
-    return v;
-}
 
 static_assert(kLayoutSlots == 64, "one layout statistics slot per lane");
 
@@ -1231,185 +1225,6 @@ __global__ void __launch_bounds__(64 * NW, NW * AP == 8 ? 1 : 2) k_conv_mfma_wre
     }
 }
 
-// ---------------------------------------------------------------------------
-// Output-stationary MFMA kernel for Ci = 64 (bf16 / fp16 storage).
-//
-// The compacted kernels add each 128-pair unit's products into fp32 tile sums
-// in LDS; with Ci = 64 a unit is only two K steps, so that read-modify-write
-// (Co x 8 bytes per pair) costs more than the unit's MFMAs.  Here every row's
-// sums stay in registers for all 27 offsets: a block owns one 256-row map
-// tile (4 wavefronts x 64 rows, lane = row), a wavefront 4 row blocks of 16
-// x all Co = 64 channels.  For offset k each row's source is read from the
-// tile's pair list for k (its rank among the tile's rows with a neighbour at
-// k comes from ballots of the row masks), and the 16 source rows of a row
-// block are loaded straight into MFMA operand order (lane i + 16 c: chunk c
-// of row i's 64-byte K step); a row without a neighbour at k multiplies
-// zeros.  (Loading each row's 64 bytes with four neighbouring lanes and
-// moving them to operand order with ds_bpermute, 4 per fragment, measured
-// 15 % slower: config 4, 1.196 -> 1.036 ms.)  The loads are raw buffer loads over x: a missing neighbour gets an
-// offset past the buffer's end, which the hardware answers with zeros and no
-// memory request, so no branch guards a load and the compiler's memory waits
-// keep the two-offset look-ahead (a guarded load made it wait for each
-// offset's loads almost at once).  The offset's 8 KB of weights are shared
-// through a double-buffered LDS slot: one barrier per offset.  Each row's 27 sources are fetched in one
-// round trip at the start; operand loads run two offsets ahead.  No unit
-// lists, no tile sums, no flushes: the MFMA rows include the rows without a
-// neighbour (27 N row-offsets against P), which is the price of keeping the
-// sums in registers.  (Sorting each tile's rows by mask, so that 16-row
-// blocks without a neighbour at k could be skipped, measured slower.)
-// ---------------------------------------------------------------------------
-template <int DT>
-__global__ void __launch_bounds__(256, 2) k_conv_os64(const typename Store<DT>::T * __restrict__ x,
-                                                      const int32_t * __restrict__ pair_src,
-                                                      const int32_t * __restrict__ tile_off,
-                                                      const uint32_t * __restrict__ mask,
-                                                      const typename Store<DT>::T * __restrict__ w16,
-                                                      const float * __restrict__ bias,
-                                                      typename Store<DT>::T * __restrict__ y, int64_t n) {
-    using T = typename Store<DT>::T;
-    using V = typename Mfma<DT>::V;
-    constexpr int CI = 64, CO = 64;
-    // The weights come in conv_stream_group(64, 64)'s packing, which this
-    // kernel reads with g = 4: lane l16 owns channels 4 l16 .. 4 l16 + 3.
-    static_assert(64 / (TSH_STREAM_WAVES / TSH_STREAM_ROW_GROUPS) / 16 == 4,
-                  "k_conv_os64 needs the 64-channel grouped packing with g = 4");
-    constexpr int QB = 4;                      // row blocks per wavefront
-    constexpr int NT = CO / 16;                // column tiles (grouped packing: lane's NT columns adjacent)
-    constexpr int WSLOT = (CI / 8) * CO * 8;   // weight elements per offset
-    constexpr int WPT = WSLOT * 2 / 16 / 256;  // 16-byte weight pieces per thread per offset
-    static_assert(WPT == 2, "8 KB of weights per offset over 256 threads");
-    __shared__ __attribute__((aligned(16))) T s_w[2][WSLOT];
-    __shared__ int32_t s_cnt[27][4];
-    __shared__ int32_t s_off[27];
-
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wave = t >> 6;
-    const int l16 = lane & 15, lg = lane >> 4;
-    const int64_t tile = xcd_remap(blockIdx.x, (int64_t) gridDim.x);
-    const int64_t row0 = tile * kMapTile;
-    const int64_t my_row = row0 + wave * 64 + lane;
-    const uint32_t m = my_row < n ? mask[my_row] : 0u;
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    if (t < 27) s_off[t] = tile_off[tile * 27 + t];
-    // Rows of each wavefront with a neighbour at k, for the ranks below.
-#pragma unroll 1
-    for (int k = 0; k < 27; ++k) {
-        const int c = __popcll(__ballot((m >> k) & 1u));
-        if (lane == 0) s_cnt[k][wave] = c;
-    }
-    // Weights of offsets 0 (into slot 0) and 1 (in registers).
-    V wreg[WPT];
-#pragma unroll
-    for (int j = 0; j < WPT; ++j) wreg[j] = *(const V *) (w16 + (int64_t) (t + j * 256) * 8);
-#pragma unroll
-    for (int j = 0; j < WPT; ++j) *(V *) &s_w[0][(t + j * 256) * 8] = wreg[j];
-#pragma unroll
-    for (int j = 0; j < WPT; ++j) wreg[j] = *(const V *) (w16 + WSLOT + (int64_t) (t + j * 256) * 8);
-    lds_barrier();
-
-    // Source rows of this lane's row at every offset (or -1), all fetched
-    // in one round trip: the row's rank in the tile's list for k is the
-    // count of earlier rows with a neighbour at k.
-    int32_t src[27];
-#pragma unroll
-    for (int k = 0; k < 27; ++k) {
-        const uint64_t bk = __ballot((m >> k) & 1u);
-        int base = 0;
-        for (int w = 0; w < wave; ++w) base += s_cnt[k][w];
-        src[k] = ((m >> k) & 1u) ? pair_src[s_off[k] + base + __popcll(bk & lt)] : -1;
-    }
-    // A fragments of offset k: row block q, K step f; lane i + 16 c holds 16
-    // bytes (chunk c of the step) of row i of the block.  Byte offsets into x
-    // per row block, prepared one offset before their loads so that the
-    // shuffles' latency stays off the load path.
-    constexpr int AHEAD = 2;  // offsets whose A loads are in flight
-    const __amdgpu_buffer_rsrc_t xres =
-        __builtin_amdgcn_make_buffer_rsrc((void *) x, 0, (int) (n * CI * (int64_t) sizeof(T)), 0x00020000);
-    V ra[AHEAD + 1][QB][2];
-    uint32_t voff[QB];
-    auto prep_a = [&](int32_t src) {
-#pragma unroll
-        for (int q = 0; q < QB; ++q) {
-            const int32_t sq = __shfl(src, q * 16 + l16);
-            voff[q] = sq >= 0 ? (uint32_t) sq * (uint32_t) (CI * sizeof(T)) + (uint32_t) lg * 16u : 0x80000000u;
-        }
-    };
-    auto load_a = [&](V (&a)[QB][2]) {
-#pragma unroll
-        for (int q = 0; q < QB; ++q)
-#pragma unroll
-            for (int f = 0; f < 2; ++f)
-                a[q][f] = __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(xres, voff[q] + f * 64u, 0, 0));
-    };
-    f32x4 acc[QB][NT];
-#pragma unroll
-    for (int q = 0; q < QB; ++q)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[q][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < AHEAD; ++k) {
-        prep_a(src[k]);
-        load_a(ra[k]);
-    }
-    prep_a(src[AHEAD]);
-#pragma unroll
-    for (int k = 0; k < 27; ++k) {
-        const int cur = k & 1;
-        const int ar = k % (AHEAD + 1);
-        if (k + AHEAD < 27) load_a(ra[(k + AHEAD) % (AHEAD + 1)]);
-        if (k + AHEAD + 1 < 27) prep_a(src[k + AHEAD + 1]);
-        // Keeps the loads just issued ahead of this offset's weight reads and
-        // MFMAs (the scheduler would interleave them).
-        __builtin_amdgcn_sched_barrier(0);
-        // Weight fragments of offset k: K step f, column tile nt.
-        V bw[2][NT];
-        const T * ws = &s_w[cur][0];
-#pragma unroll
-        for (int f = 0; f < 2; ++f)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) bw[f][nt] = *(const V *) (ws + ((f * 4 + lg) * CO + nt * 16 + l16) * 8);
-#pragma unroll
-        for (int q = 0; q < QB; ++q)
-#pragma unroll
-            for (int f = 0; f < 2; ++f) {
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc[q][nt] = Mfma<DT>::mac(ra[ar][q][f], bw[f][nt], acc[q][nt]);
-            }
-        // Offset k + 1's weights into the other slot (read last at offset
-        // k - 1, before the previous barrier); offset k + 2's into registers.
-        if (k + 1 < 27) {
-#pragma unroll
-            for (int j = 0; j < WPT; ++j) *(V *) &s_w[cur ^ 1][(t + j * 256) * 8] = wreg[j];
-        }
-        if (k + 2 < 27) {
-#pragma unroll
-            for (int j = 0; j < WPT; ++j)
-                wreg[j] = *(const V *) (w16 + (int64_t) (k + 2) * WSLOT + (int64_t) (t + j * 256) * 8);
-        }
-        lds_barrier();
-    }
-    // Epilogue: bias, round, store; lane holds rows 4 lg + i of each row
-    // block, channels 4 l16 .. 4 l16 + 3 (grouped packing).
-    float bv[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) bv[nt] = bias != nullptr ? bias[l16 * NT + nt] : 0.0f;
-#pragma unroll
-    for (int q = 0; q < QB; ++q)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t row = row0 + wave * 64 + q * 16 + lg * 4 + i;
-            if (row >= n) continue;
-            union {
-                uint2 u;
-                T h[4];
-            } o;
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) o.h[nt] = round_to_store<DT>(acc[q][nt][i] + bv[nt]);
-            *(uint2 *) (y + row * CO + l16 * NT) = o.u;
-        }
-}
-
 }  // namespace
 
 hipError_t launch_conv_generic(int dtype, const void * x, const int32_t * nbr, const float * w32, const float * bias,
@@ -1585,29 +1400,6 @@ hipError_t launch_stream_dt(const void * x, const int32_t * pair_src, const uint
 #undef TSH_STREAM
 }
 }  // namespace
-
-// The gathers address x through a buffer resource whose byte range is an
-// int32: up to 2^31 / 128 rows (16.7M voxels); beyond that the compacted
-// streamed kernel runs instead.
-bool conv_os_supported(int dtype, int ci, int co, int64_t n) {
-    return (dtype == kF16 || dtype == kBF16) && ci == 64 && co == 64 && n > 0 && n <= (int64_t) INT32_MAX / 128;
-}
-
-hipError_t launch_conv_os(int dtype, const void * x, const int32_t * pair_src, const int32_t * tile_off,
-                          const uint32_t * mask, const void * w16, const float * bias, void * y, int64_t n, int ci,
-                          int co, hipStream_t s) {
-    if (!conv_os_supported(dtype, ci, co, n)) return hipErrorInvalidValue;
-    const int64_t tiles = (n + kMapTile - 1) / kMapTile;
-    if (tiles > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (dtype == kBF16) {
-        k_conv_os64<kBF16><<<(unsigned) tiles, 256, 0, s>>>((const uint16_t *) x, pair_src, tile_off, mask,
-                                                            (const uint16_t *) w16, bias, (uint16_t *) y, n);
-    } else {
-        k_conv_os64<kF16><<<(unsigned) tiles, 256, 0, s>>>((const _Float16 *) x, pair_src, tile_off, mask,
-                                                           (const _Float16 *) w16, bias, (_Float16 *) y, n);
-    }
-    return hipGetLastError();
-}
 
 hipError_t launch_conv_mfma_stream(int dtype, const void * x, const int32_t * pair_src, const uint8_t * pair_dst,
                                    const int32_t * tile_off, const int32_t * tile_counts, const uint32_t * mask,

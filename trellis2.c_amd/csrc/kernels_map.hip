@@ -13,8 +13,10 @@
 //   voxel pool   int32 [bricks][64]: row of the voxel at cell (z&3)|(y&3)<<2|(x&3)<<4, -1 = empty
 //                (z fastest: a 16-byte load returns a voxel's z-row, the three
 //                cells of a (kd, kh) stencil column for cells off the z faces).
-//   nbr          int32 [n][27]
-//   mask         uint32 [n], bit k <=> nbr[i][k] >= 0
+//   rows         int32 [n][28]: a row's 27 neighbour rows (-1 = none), then its mask; 112 bytes, so that one
+//                lane writes and reads a row in 16-byte pieces
+//   mask         uint32 [n], bit k <=> rows[i][k] >= 0
+// Pair lists (written from the rows for the kernels that walk them):
 //   tile_counts  int32 [n_tiles][27] valid pairs per 256-row tile and offset
 //   pairs        tile-major: tile t's lists for offset k start at tile_off[t][k] (tiles ascending,
 //                offsets ascending within a tile, dst ascending within an offset); pair_src int32
@@ -210,47 +212,19 @@ __global__ void __launch_bounds__(kBlock) k_voxel_insert(const int4 * __restrict
     atomicMax(&pool[(int64_t) b * kBrickCells + cell], (int32_t) i);
 }
 
-// Kernel map in one pass.  One block = one 256-row tile:
-//  1. each row's 27 neighbour rows are found (a few brick probes per voxel
-//     plus 9 z-row pool reads) and kept in its lane's registers, with the row
-//     masks; only a launch that also writes the neighbour table (NBR) stages
-//     the tile's [256][27] rows in LDS, for a coalesced copy.  Without that
-//     28 KB of LDS per block the kernel runs 8 wavefronts per SIMD instead
-//     of 5, which is what its dependent probe and pool loads need;
-//  2. per-offset pair counts of the tile (wavefront ballots);
-//  3. the neighbour table (16-byte vectorised copy of the LDS block), the
-//     per-(tile, offset) counts and list starts, and the pair lists,
-//     destination ascending within each (tile, offset).
-// Tile t owns the fixed region [t * 256 * 27, (t + 1) * 256 * 27) of the
-// pair arrays (the most pairs 256 rows can have), so no tile waits for the
-// counts of the tiles before it; the lists of a tile are packed from the
-// region's start, the centre offset (k = 13) first, then the others in
-// order.  Every row has exactly one centre neighbour (itself, or the last
-// duplicate of its coordinates), so the centre list holds the tile's rows in
-// order, starting at the region's start: a consumer can find it without the
-// tile's counts.
+// Kernel map: one lane finds its voxel's 27 neighbour rows (a few brick probes
+// plus 9 z-row pool reads), keeps them in registers and writes them with the
+// row mask as seven 16-byte pieces.  (Until the convs read this table, the
+// kernel packed per-tile pair lists instead, which took 27 ballots, ranks and
+// scattered stores per wavefront.)
 // Seven wavefronts per SIMD (at most 72 registers): 4 % faster than six on
-// config 3's map, while eight spill.  The launch that also writes the
-// neighbour table holds 28 KB of LDS per block, which allows five.
-template <bool NBR>
-__global__ void __launch_bounds__(kBlock, NBR ? 5 : 7) k_map_tiles(const int4 * __restrict__ coords, int64_t n,
-                                                      const uint64_t * __restrict__ table, uint64_t hmask,
-                                                      const int32_t * __restrict__ pool, int32_t empty_brick,
-                                                      int32_t * __restrict__ nbr,
-                                                      uint32_t * __restrict__ mask_out,
-                                                      int32_t * __restrict__ tile_counts,
-                                                      int32_t * __restrict__ tile_off,
-                                                      int32_t * __restrict__ pair_src,
-                                                      uint8_t * __restrict__ pair_dst, int32_t * __restrict__ counters) {
-    __shared__ __attribute__((aligned(16))) int32_t s_nbr[NBR ? kBlock * 27 : 4];
-    __shared__ int32_t s_wave_cnt[27][kBlock / 64];
-    __shared__ int32_t s_koff[27];
-    const int t = threadIdx.x;
-    const int lane = lane_id();
-    const int wave = t >> 6;
-    const int64_t tile = blockIdx.x;
-    const int64_t row0 = tile * kBlock;
-    const int64_t i = row0 + t;
+// config 3's map, while eight spill.
+__global__ void __launch_bounds__(kBlock, 7) k_map_rows(const int4 * __restrict__ coords, int64_t n,
+                                                        const uint64_t * __restrict__ table, uint64_t hmask,
+                                                        const int32_t * __restrict__ pool, int32_t empty_brick,
+                                                        int32_t * __restrict__ rows, uint32_t * __restrict__ mask_out,
+                                                        int32_t * __restrict__ counters) {
+    const int64_t i = (int64_t) blockIdx.x * kBlock + threadIdx.x;
     uint32_t m = 0;
     int32_t nb[27];
 #pragma unroll
@@ -335,14 +309,57 @@ __global__ void __launch_bounds__(kBlock, NBR ? 5 : 7) k_map_tiles(const int4 * 
                 const int32_t r = nz < 0 || nz > 3 ? e : (nz == 0 ? v.x : (nz == 1 ? v.y : (nz == 2 ? v.z : v.w)));
                 const int k = c * 3 + kw;
                 nb[k] = r;
-                if constexpr (NBR) s_nbr[t * 27 + k] = r;
                 m |= (r >= 0 ? 1u : 0u) << k;
             }
         }
         mask_out[i] = m;
+        int4 * out = (int4 *) (rows + i * kMapRow);
+#pragma unroll
+        for (int c = 0; c < 6; ++c) out[c] = int4{nb[4 * c], nb[4 * c + 1], nb[4 * c + 2], nb[4 * c + 3]};
+        out[6] = int4{nb[24], nb[25], nb[26], (int32_t) m};
         // The centre neighbour is the highest row at these coordinates: any
         // other value means duplicate coordinates.
         if (nb[13] != (int32_t) i) atomicOr(&counters[1], 1);
+    }
+}
+
+// Per-tile pair lists from the row table; one block = one 256-row tile:
+//  1. per-offset pair counts of the tile (wavefront ballots);
+//  2. the per-(tile, offset) counts and list starts, and the pair lists,
+//     destination ascending within each (tile, offset).
+// Tile t owns the fixed region [t * 256 * 27, (t + 1) * 256 * 27) of the
+// pair arrays (the most pairs 256 rows can have), so no tile waits for the
+// counts of the tiles before it; the lists of a tile are packed from the
+// region's start, the centre offset (k = 13) first, then the others in
+// order.  Every row has exactly one centre neighbour (itself, or the last
+// duplicate of its coordinates), so the centre list holds the tile's rows in
+// order, starting at the region's start: a consumer can find it without the
+// tile's counts.
+__global__ void __launch_bounds__(kBlock) k_map_lists(const int32_t * __restrict__ rows, int64_t n,
+                                                      int32_t * __restrict__ tile_counts,
+                                                      int32_t * __restrict__ tile_off,
+                                                      int32_t * __restrict__ pair_src,
+                                                      uint8_t * __restrict__ pair_dst, int32_t * __restrict__ counters) {
+    __shared__ int32_t s_wave_cnt[27][kBlock / 64];
+    __shared__ int32_t s_koff[27];
+    const int t = threadIdx.x;
+    const int lane = lane_id();
+    const int wave = t >> 6;
+    const int64_t tile = blockIdx.x;
+    const int64_t i = tile * kBlock + t;
+    uint32_t m = 0;
+    int32_t nb[28];
+    if (i < n) {
+        const int4 * in = (const int4 *) (rows + i * kMapRow);
+#pragma unroll
+        for (int c = 0; c < 7; ++c) {
+            const int4 v = in[c];
+            nb[4 * c] = v.x;
+            nb[4 * c + 1] = v.y;
+            nb[4 * c + 2] = v.z;
+            nb[4 * c + 3] = v.w;
+        }
+        m = (uint32_t) nb[27];
     }
     // Rows of this wavefront with a neighbour at k (the ranks are recomputed
     // from the same ballots when the pairs are written).
@@ -383,21 +400,6 @@ __global__ void __launch_bounds__(kBlock, NBR ? 5 : 7) k_map_tiles(const int4 * 
     __syncthreads();
     const int64_t base = tile * kBlock * 27;
     if (t < 27) tile_off[tile * 27 + t] = (int32_t) (base + s_koff[t]);
-    if constexpr (NBR) {
-        // Coalesced copy of the tile's neighbour table.
-        const int64_t rows = (n - row0) < kBlock ? (n - row0) : kBlock;
-        const int64_t words = rows * 27;
-        int32_t * dst = nbr + row0 * 27;
-        if ((words & 3) == 0) {
-            for (int64_t w = (int64_t) t * 4; w < words; w += kBlock * 4) {
-                *(int4 *) (dst + w) = *(const int4 *) (s_nbr + w);
-            }
-        } else {
-            for (int64_t w = t; w < words; w += kBlock) {
-                dst[w] = s_nbr[w];
-            }
-        }
-    }
     // Every lane takes part in the ballots; rows past n have no neighbours.
 #pragma unroll
     for (int k = 0; k < 27; ++k) {
@@ -454,21 +456,32 @@ hipError_t launch_voxel_insert(const int32_t * coords, int64_t n, const uint64_t
     return hipGetLastError();
 }
 
-hipError_t launch_map_tiles(const int32_t * coords, int64_t n, const uint64_t * table,
-                            int64_t slots, const int32_t * pool, int32_t * nbr, uint32_t * mask,
-                            int32_t * tile_counts, int32_t * tile_off, int32_t * pair_src, uint8_t * pair_dst,
-                            int32_t * counters, hipStream_t s) {
+hipError_t launch_map_rows(const int32_t * coords, int64_t n, const uint64_t * table, int64_t slots,
+                           const int32_t * pool, int32_t * rows, uint32_t * mask, int32_t * counters, hipStream_t s) {
     const int64_t blocks = (n + kBlock - 1) / kBlock;
-    const int32_t empty = (int32_t) pool_empty_brick(n);
-    if (nbr != nullptr) {
-        k_map_tiles<true><<<(unsigned) blocks, kBlock, 0, s>>>((const int4 *) coords, n, table,
-                                                               (uint64_t) (slots - 1), pool, empty, nbr, mask,
-                                                               tile_counts, tile_off, pair_src, pair_dst, counters);
-    } else {
-        k_map_tiles<false><<<(unsigned) blocks, kBlock, 0, s>>>((const int4 *) coords, n, table,
-                                                                (uint64_t) (slots - 1), pool, empty, nbr, mask,
-                                                                tile_counts, tile_off, pair_src, pair_dst, counters);
+    k_map_rows<<<(unsigned) blocks, kBlock, 0, s>>>((const int4 *) coords, n, table, (uint64_t) (slots - 1), pool,
+                                                    (int32_t) pool_empty_brick(n), rows, mask, counters);
+    return hipGetLastError();
+}
+
+hipError_t launch_map_lists(const int32_t * rows, int64_t n, int32_t * tile_counts, int32_t * tile_off,
+                            int32_t * pair_src, uint8_t * pair_dst, int32_t * counters, hipStream_t s) {
+    const int64_t blocks = (n + kBlock - 1) / kBlock;
+    k_map_lists<<<(unsigned) blocks, kBlock, 0, s>>>(rows, n, tile_counts, tile_off, pair_src, pair_dst, counters);
+    return hipGetLastError();
+}
+
+// The dense [n][27] neighbour table of the row table.
+__global__ void k_rows_nbr(const int32_t * __restrict__ rows, int64_t n, int32_t * __restrict__ nbr) {
+    const int64_t stride = (int64_t) gridDim.x * blockDim.x;
+    for (int64_t e = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; e < n * 27; e += stride) {
+        const int64_t i = e / 27;
+        nbr[e] = rows[i * kMapRow + (e - i * 27)];
     }
+}
+
+hipError_t launch_rows_nbr(const int32_t * rows, int64_t n, int32_t * nbr, hipStream_t s) {
+    k_rows_nbr<<<grid_for(n * 27, 256, 16384), 256, 0, s>>>(rows, n, nbr);
     return hipGetLastError();
 }
 

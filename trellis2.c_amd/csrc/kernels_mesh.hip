@@ -81,7 +81,7 @@ __device__ inline bool fdg_quad(const typename Store<DT>::T * f, const int32_t *
     bool ok = true;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        q[j] = nbr[i * 27 + kQuadK[a][j]];
+        q[j] = nbr[i * kMapRow + kQuadK[a][j]];
         ok &= q[j] >= 0;
     }
     return ok;

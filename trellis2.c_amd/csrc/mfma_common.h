@@ -86,5 +86,15 @@ __device__ __forceinline__ int a_granule(int i, int c) {
 }
 __device__ __forceinline__ int a_quad_row(int j) { return (j & 5) | (((j >> 1) & 1) << 3) | (((j >> 3) & 1) << 1); }
 
+// Sum over the 16 lanes of a DPP row, left in every lane of the row:
+// rotations by 8, 4, 2 and 1 within the row (row_ror), each one VALU add.
+__device__ __forceinline__ float row16_sum(float v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x124, 0xf, 0xf, false));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x122, 0xf, 0xf, false));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false));
+    return v;
+}
+
 }  // namespace
 }  // namespace tsh

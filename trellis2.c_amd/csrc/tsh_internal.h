@@ -104,6 +104,7 @@ template <int DT> __device__ inline int4 pack_chunk(const float * v) {
 
 // Work split of a rulebook build / conv: rows per tile of the kernel map.
 constexpr int kMapTile = 256;
+constexpr int kMapRow = 28;      // words of a row of the kernel map: 27 neighbour rows and the mask
 constexpr int kBrickCells = 64;  // 4x4x4 cells per brick
 // Build counters: [1] duplicate flag, [4] internal-error flags, the brick
 // count (statistics) summed over kBrickCounters counters from
@@ -147,13 +148,16 @@ struct trellis_sparse_rulebook {
     tsh::DevMem pool;        // int32  [cap_bricks][64] voxel rows, -1 = empty
     tsh::DevMem counters;    // int32  [kCounterInts]: [1] duplicate flag, [4] internal-error flags, [64..] brick counts, [128..] layout statistics
     // Kernel map.
-    tsh::DevMem nbr;         // int32  [n][27]
-    tsh::DevMem mask;        // uint32 [n] bit k set when nbr[i][k] >= 0
+    tsh::DevMem rows;        // int32  [n][kMapRow]: 27 neighbour rows (-1 = none), then the mask
+    tsh::DevMem mask;        // uint32 [n] bit k set when rows[i][k] >= 0
     int64_t n_tiles;         // ceil(n / kMapTile)
+    // Pair lists (built for the kernels that walk them).
     tsh::DevMem tile_counts; // int32  [n_tiles][27]
     tsh::DevMem tile_off;    // int32  [n_tiles][27] start of (tile, k) in the pair arrays
     tsh::DevMem pair_src;    // int32  [n_tiles][kMapTile * 27]: per tile, offsets ascending, dst ascending
     tsh::DevMem pair_dst;    // uint8  [n_tiles][kMapTile * 27]: destination row within the tile
+    // Mask order (built by the first conv that takes the rows in it).
+    tsh::DevMem perm;        // int32  [n] row at each place
 };
 
 struct trellis_sparse_c2s_device_map {
@@ -188,13 +192,27 @@ int64_t pool_empty_brick(int64_t n);
 
 hipError_t launch_voxel_insert(const int32_t * coords, int64_t n, const uint64_t * table,
                                int64_t slots, int32_t * pool, int32_t * counters, hipStream_t s);
-// Neighbour table, masks, per-(tile, offset) counts and list starts, and the
-// pair lists in one pass.  Tile t's lists fill the start of its region
+// Neighbour rows and masks of every voxel.
+hipError_t launch_map_rows(const int32_t * coords, int64_t n, const uint64_t * table, int64_t slots,
+                           const int32_t * pool, int32_t * rows, uint32_t * mask, int32_t * counters, hipStream_t s);
+// Per-(tile, offset) counts and list starts and the pair lists from the row
+// table.  Tile t's lists fill the start of its region
 // [t * kMapTile * 27, (t + 1) * kMapTile * 27) of the pair arrays.
-hipError_t launch_map_tiles(const int32_t * coords, int64_t n, const uint64_t * table,
-                            int64_t slots, const int32_t * pool, int32_t * nbr, uint32_t * mask,
-                            int32_t * tile_counts, int32_t * tile_off, int32_t * pair_src, uint8_t * pair_dst,
-                            int32_t * counters, hipStream_t s);
+hipError_t launch_map_lists(const int32_t * rows, int64_t n, int32_t * tile_counts, int32_t * tile_off,
+                            int32_t * pair_src, uint8_t * pair_dst, int32_t * counters, hipStream_t s);
+// The dense [n][27] neighbour table of the row table.
+hipError_t launch_rows_nbr(const int32_t * rows, int64_t n, int32_t * nbr, hipStream_t s);
+
+// Mask order of a rulebook's rows (kernels_order.hip): perm[place] = row,
+// sorted within windows of `window` rows (a multiple of 4096).  bins:
+// order_bins_bytes of scratch.  Larger windows fill blocks better, smaller
+// ones keep a block's sources closer together; measured on 0.4-3.8 million
+// rows, 2^18 is the best or within 2 % (3,788,747 rows, 64 -> 64: 0.85 ms,
+// 0.91 in one window, 0.86 with 2^16, 0.91 with 2^14, 1.04 in row order).
+constexpr int64_t kOrderWindow = 1 << 18;
+size_t order_bins_bytes(int64_t n, int64_t window);
+hipError_t launch_order(const uint32_t * mask, int64_t n, int64_t window, int32_t * bins, int32_t * perm,
+                        hipStream_t s);
 
 // Convolution (kernels_conv.hip).  Weight layouts are produced by the backend.
 //  generic: w32 fp32 [27][ci][co]
@@ -235,12 +253,13 @@ hipError_t launch_conv_mfma_stream(int dtype, const void * x, const int32_t * pa
                                    const void * w16, const float * bias, void * y, int64_t n, int ci, int co,
                                    hipStream_t s, const ConvEpilogue & epi, const int32_t * layout_stats);
 
-// Output-stationary MFMA conv for Ci = Co = 64 over the tile-major pair lists
-// and the row masks (weights in the grouped packing of conv_stream_group(64, 64)).
-bool conv_os_supported(int dtype, int ci, int co, int64_t n);
-hipError_t launch_conv_os(int dtype, const void * x, const int32_t * pair_src, const int32_t * tile_off,
-                          const uint32_t * mask, const void * w16, const float * bias, void * y, int64_t n, int ci,
-                          int co, hipStream_t s);
+// Output-stationary MFMA conv over rows in mask order (kernels_conv_sorted.hip),
+// or in their own order with perm == nullptr; weights in the grouped packing
+// of conv_stream_group(ci, co).
+bool conv_sorted_supported(int dtype, int ci, int co, int64_t n);
+hipError_t launch_conv_sorted(int dtype, const void * x, const int32_t * rows, const int32_t * perm, const void * w16,
+                              const float * bias, void * y, int64_t n, int ci, int co, int cus, hipStream_t s,
+                              const ConvEpilogue & epi);
 
 // Everything else (kernels_misc.hip).
 hipError_t launch_convert_from_f32(int dtype, const float * src, void * dst, int64_t count, hipStream_t s);
