@@ -57,7 +57,8 @@ enum WeightLayout : int {
     kLayoutLinearMfma = 6,       // storage type [ci/8][co][8], linear_mfma_group column grouping
     kLayoutMlp0 = 7,             // as kLayoutLinearMfma, the fused MLP's first GEMM grouping
     kLayoutMlp2 = 8,             // as kLayoutLinearMfma, the fused MLP's second GEMM grouping
-    kLayoutLinear16 = 9          // storage type [co][ci] (narrow MFMA linear)
+    kLayoutLinear16 = 9,         // storage type [co][ci] (narrow MFMA linear)
+    kLayoutGemm = 10             // as kLayoutLinearMfma, groups of 128 columns, 8 adjacent channels per lane
 };
 
 struct StageMark {
@@ -453,12 +454,15 @@ trellis_status get_weight(Backend * be, const float * host, size_t count, int la
             break;
         }
         case kLayoutLinearMfma:  // [co][ci] -> [ci/8][co][8] in the storage type, grouped columns
+        case kLayoutGemm:
         case kLayoutMlp0:
         case kLayoutMlp2: {
             staged.resize((size_t) ci * co * 2);
             uint16_t * w = (uint16_t *) staged.data();
             int g = linear_mfma_group(co);
-            if (layout != kLayoutLinearMfma) {
+            if (layout == kLayoutGemm) {
+                g = 8;
+            } else if (layout != kLayoutLinearMfma) {
                 int g0 = 1, g2 = 1;
                 convnext_mlp_groups(layout == kLayoutMlp0 ? ci : co, &g0, &g2);
                 g = layout == kLayoutMlp0 ? g0 : g2;
@@ -637,7 +641,8 @@ void op_free_buffer(trellis_sparse_backend * backend, trellis_sparse_buffer * bu
 
 // y = x W^T + b (then SiLU).  With a residual (no SiLU): y = residual +
 // (x W^T + b), residual [n][co] (may be y): the GEMM library adds it to the
-// fp32 sums before the one rounding; the kernels write the rounded linear
+// fp32 sums before the one rounding; the GEMM kernel adds it to the rounded
+// linear output in its epilogue; the other kernels write the rounded linear
 // output to scratch ([n][co], neither y nor residual) and the add kernel
 // forms the sum.
 trellis_status linear_impl(trellis_sparse_backend * backend, const trellis_sparse_buffer * x, const float * weight,
@@ -656,9 +661,10 @@ trellis_status linear_impl(trellis_sparse_backend * backend, const trellis_spars
     const void * wt = nullptr;
     const void * bd = nullptr;
     const int dt = be->policy.compute_dtype;
-    // bf16/fp16 with Ci = 64 or Ci % 128 == 0 and Co % 64 == 0: MFMA kernel;
-    // Co <= 16 (the subdivide logits): the narrow MFMA kernel; otherwise (and
-    // always for fp32) the reference-order VALU kernel.
+    // bf16/fp16 with Ci % 64 == 0 and Co % 128 == 0: the GEMM kernel; Ci = 64
+    // or Ci % 128 == 0 and other Co % 64 == 0: the MFMA linear kernel; Co <= 16
+    // (the subdivide logits): the narrow MFMA kernel; otherwise (and always
+    // for fp32) the reference-order VALU kernel.
     trellis_status st = get_weight(be, bias, (size_t) co, kLayoutVector, 0, co, &bd);
     if (st != TRELLIS_STATUS_OK) return st;
     // Wide shapes: the platform GEMM library when it has a plan (workspace
@@ -681,6 +687,15 @@ trellis_status linear_impl(trellis_sparse_backend * backend, const trellis_spars
             stage_end(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
             if (done) return TRELLIS_STATUS_OK;
         }
+    }
+    if (gemm_supported(dt, n, ci, co)) {
+        st = get_weight(be, weight, (size_t) ci * co, kLayoutGemm, ci, co, &wt);
+        if (st != TRELLIS_STATUS_OK) return st;
+        stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
+        const hipError_t err = launch_gemm(dt, x->ptr, wt, (const float *) bd, residual ? residual->ptr : nullptr,
+                                           y->ptr, n, ci, co, silu, be->cus, be->stream);
+        stage_end(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
+        return hip_status(be, err, "linear");
     }
     const bool mfma = linear_mfma_supported(dt, ci, co);
     const bool narrow = !mfma && linear_narrow_supported(dt, ci, co);

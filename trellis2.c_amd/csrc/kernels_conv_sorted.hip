@@ -2,7 +2,7 @@
 #include <type_traits>
 
 #include "tsh_internal.h"
-#include "mfma_common.h"
+#include "mfma_ring.h"
 
 namespace tsh {
 namespace {
@@ -52,15 +52,8 @@ __global__ void __launch_bounds__(64 * RW * CW, RW * CW == 8 ? 2 : 1)
     constexpr int QB = BM / RW / 16;   // row blocks per wavefront
     constexpr int NT = BN / CW / 16;   // column tiles per wavefront
     constexpr int NA = BM / 16 / NW;   // A loads per wavefront and step (16 rows each)
-    // Weight loads per wavefront and step (1 KB each, 64 16-byte granules);
-    // with fewer loads than wavefronts some fetch the same ones, so that
-    // every wavefront counts the same number of outstanding loads.
-    constexpr int WL = BN / 16;
-    constexpr int NB = WL < NW ? 1 : WL / NW;
-    constexpr int PER = NA + NB;
-    constexpr int SLOT = (BM + BN) * 64;
-    static_assert(NA >= 1 && BM % (16 * NW) == 0 && (WL % NW == 0 || NW % WL == 0), "whole loads");
-    static_assert(QB >= 1 && NT >= 1 && BM % (16 * RW) == 0 && BN % (16 * CW) == 0, "whole MFMA tiles");
+    using R = RingShape<BM, BN, RW, CW>;
+    constexpr int WL = R::WL, NB = R::NB, SLOT = R::SLOT;  // weight loads of a step: the block's, a wavefront's
     constexpr int OUT = BM * BN * 2;
     constexpr int RING = SLOTS * SLOT > OUT ? SLOTS * SLOT : OUT;
     __shared__ __attribute__((aligned(1024))) unsigned char s_ring[RING];
@@ -173,122 +166,10 @@ __global__ void __launch_bounds__(64 * RW * CW, RW * CW == 8 ? 2 : 1)
         }
     };
 
-    // ---- fragments ------------------------------------------------------
-    const uint32_t a_at = (uint32_t) (rw * QB * 1024 + (l16 * 4 + (lg ^ ((l16 >> 3) << 1))) * 16);
-    const uint32_t b_at = (uint32_t) (BM * 64 + (lg * BN + cw * NT * 16 + l16) * 16);
-    V fa[2][QB], fb[2][NT];
     f32x4 acc[QB][NT];
-#pragma unroll
-    for (int q = 0; q < QB; ++q)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[q][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
     fetch_src();
     next_offset();
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s) {
-#pragma unroll
-        for (int j = 0; j < PER; ++j) load(j);
-        advance();
-    }
-    uint32_t rslot = 0;  // slot offset of the step whose fragments are read next
-    if constexpr (PP) {
-        static_assert(!PP || NW == 8, "two wavefronts per SIMD");
-        // Phases alternate at barriers; a slot is refilled once both halves
-        // have read it.
-        auto mem = [&](bool issue) {
-#pragma unroll
-            for (int q = 0; q < QB; ++q) fa[0][q] = *(const V *) (s_ring + rslot + a_at + q * 1024);
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) fb[0][nt] = *(const V *) (s_ring + rslot + b_at + nt * 256);
-            if (issue) {
-#pragma unroll
-                for (int j = 0; j < PER; ++j) load(j);
-                advance();
-            }
-            rslot = rslot == (SLOTS - 1) * SLOT ? 0 : rslot + SLOT;
-        };
-        auto mm = [&]() {
-            __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-            for (int q = 0; q < QB; ++q)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc[q][nt] = Mfma<DT>::mac(fa[0][q], fb[0][nt], acc[q][nt]);
-            __builtin_amdgcn_s_setprio(0);
-        };
-        wait_vmcnt<(SLOTS - 1) * PER>();
-        lds_barrier();
-        const bool second = wave >= NW / 2;
-        if (second) {
-            lds_barrier();
-            for (int s = 0; s < steps; ++s) {
-                mem(s > 0);
-                wait_vmcnt<(SLOTS - 2) * PER>();
-                lds_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-                mm();
-                __builtin_amdgcn_sched_barrier(0);
-                lds_barrier();
-            }
-        } else {
-            for (int s = 0; s < steps; ++s) {
-                mem(s > 0);
-                lds_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-                mm();
-                __builtin_amdgcn_sched_barrier(0);
-                wait_vmcnt<(SLOTS - 2) * PER>();
-                lds_barrier();
-            }
-            lds_barrier();
-        }
-    } else {
-    auto read_a = [&](int p, int q) { fa[p][q] = *(const V *) (s_ring + rslot + a_at + q * 1024); };
-    auto read_b = [&](int p, int nt) { fb[p][nt] = *(const V *) (s_ring + rslot + b_at + nt * 256); };
-    wait_vmcnt<(SLOTS - 1) * PER>();
-    lds_barrier();
-#pragma unroll
-    for (int q = 0; q < QB; ++q) read_a(0, q);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) read_b(0, nt);
-    rslot = SLOT;
-
-    // One K step: fragments p hold step s; step s + 1's are read, step
-    // s + SLOTS's rows and weights go into step s's slot (every wavefront
-    // read its fragments of that slot before the barrier).
-    auto step = [&](auto pc) {
-        constexpr int p = decltype(pc)::value;
-        wait_vmcnt<(SLOTS - 2) * PER>();
-        lds_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int q = 0; q < QB; ++q) {
-            read_a(p ^ 1, q);
-            if (q < NT) read_b(p ^ 1, q);
-            if constexpr (QB < NT) {
-                if (q == QB - 1)
-#pragma unroll
-                    for (int nt = QB; nt < NT; ++nt) read_b(p ^ 1, nt);
-            }
-            if (q < PER) load(q);
-            if constexpr (QB < PER) {
-                if (q == QB - 1)
-#pragma unroll
-                    for (int j = QB; j < PER; ++j) load(j);
-            }
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[q][nt] = Mfma<DT>::mac(fa[p][q], fb[p][nt], acc[q][nt]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        advance();
-        rslot = rslot == (SLOTS - 1) * SLOT ? 0 : rslot + SLOT;
-    };
-    for (int s = 0; s < steps; s += 2) {
-        step(std::integral_constant<int, 0>());
-        step(std::integral_constant<int, 1>());
-    }
-    }
-    wait_vmcnt<0>();
+    ring_multiply<DT, BM, BN, RW, CW, SLOTS, PP>(s_ring, steps, load, advance, acc);
 
     // ---- epilogue: bias, one rounding, the tile through LDS ----------------
     // Packed column p of a group of 16 g columns holds channel (p % 16) g +

@@ -291,6 +291,12 @@ void linear_lt_destroy(LinearLt * lt);
 bool linear_lt_run(LinearLt * lt, int dtype, const void * x, const void * w16, const float * bias,
                    const void * residual, void * y, int64_t n, int ci, int co, int silu, void * workspace,
                    size_t workspace_bytes, hipStream_t s);
+// Wide linears as a GEMM through LDS (kernels_gemm.hip): 16-bit storage, Ci %
+// 64 == 0, Co % 128 == 0; the weights of launch_linear_mfma.  A non-null
+// residual (may be y) is added to the fp32 sums before the one rounding.
+bool gemm_supported(int dtype, int64_t n, int ci, int co);
+hipError_t launch_gemm(int dtype, const void * x, const void * w16, const float * bias, const void * residual,
+                       void * y, int64_t n, int ci, int co, int silu, int cus, hipStream_t s);
 // Fused ConvNeXt MLP tail (kernels_block.hip): bf16/fp16, C = 64, 128 or 256.
 // w0 [C/8][4C][8] and w2 [4C/8][C][8] in the storage type with the grouped
 // column packing of the MFMA linear, groups g0 and g2 from convnext_mlp_groups.
