@@ -346,9 +346,10 @@ hipError_t launch_dt(const void * x, const int32_t * rows, const int32_t * perm,
     if (co == 32) return TSH_SORTED(128, 32, 4, 1, 4);
     if (co % 128 != 0) {
         // 64-channel blocks: 128 rows once those fill the GPU (3,788,747
-        // rows, 64 -> 64: 0.85 ms; 5,000 rows: 0.014 against 0.010 ms).
+        // rows, 64 -> 64: 0.85 ms, 0.90 with three slots and a block less per
+        // CU; 5,000 rows: 0.014 against 0.010 ms).
         if ((n + 127) / 128 * (co / 64) < 2 * (int64_t) cus) return TSH_SORTED(64, 64, 2, 2, 4);
-        return TSH_SORTED(128, 64, 4, 1, 3);
+        return TSH_SORTED(128, 64, 4, 1, 2);
     }
     switch (pick_shape(n, ci, co, cus, epi.mode == kEpiNorm)) {
         case 0: return TSH_SORTED(256, 256, 2, 4, 4, true);

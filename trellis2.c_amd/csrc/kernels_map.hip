@@ -313,13 +313,38 @@ __global__ void __launch_bounds__(kBlock, 7) k_map_rows(const int4 * __restrict_
             }
         }
         mask_out[i] = m;
-        int4 * out = (int4 *) (rows + i * kMapRow);
-#pragma unroll
-        for (int c = 0; c < 6; ++c) out[c] = int4{nb[4 * c], nb[4 * c + 1], nb[4 * c + 2], nb[4 * c + 3]};
-        out[6] = int4{nb[24], nb[25], nb[26], (int32_t) m};
         // The centre neighbour is the highest row at these coordinates: any
         // other value means duplicate coordinates.
         if (nb[13] != (int32_t) i) atomicOr(&counters[1], 1);
+    }
+    // The rows leave through LDS, 16 of the wavefront's at a time (1.8 KB per
+    // wavefront, so that the LDS does not bound the occupancy), as
+    // consecutive 16-byte pieces; a lane writing its own row's pieces 112
+    // bytes apart took 0.276 instead of 0.229 ms on 3,788,747 rows.
+    __shared__ int4 s_rows[kBlock / 64][16 * (kMapRow / 4)];
+    const int lane = lane_id(), wave = threadIdx.x >> 6;
+    const int64_t wave0 = (int64_t) blockIdx.x * kBlock + wave * 64;
+    int4 * const stage = s_rows[wave];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        if ((lane >> 4) == g) {
+            int4 * at = stage + (lane & 15) * (kMapRow / 4);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) at[c] = int4{nb[4 * c], nb[4 * c + 1], nb[4 * c + 2], nb[4 * c + 3]};
+            at[6] = int4{nb[24], nb[25], nb[26], (int32_t) m};
+        }
+        // One wavefront's LDS operations run in order; the fence only keeps
+        // the compiler from moving them.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int64_t row0 = wave0 + g * 16;
+        const int64_t left = (n - row0) * (kMapRow / 4);
+        int4 * out = (int4 *) (rows + row0 * kMapRow);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int e = j * 64 + lane;
+            if (e < 16 * (kMapRow / 4) && e < left) out[e] = stage[e];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
 }
 
