@@ -215,6 +215,106 @@ __global__ void __launch_bounds__(256) k_conv_generic(const typename Store<DT>::
 }
 
 // ---------------------------------------------------------------------------
+// The generic order for fp32 storage with the features in scalar registers:
+// a wavefront owns R rows x 64 output channels, a lane one channel of each.
+// Per offset and 32 input channels the block's NW wavefronts share the 8 KB of
+// weights through an LDS slot (loaded straight into it two chunks ahead; each
+// wavefront fetching its own took the L2's whole rate) and a lane takes its 32
+// into registers; each of the R rows with a neighbour there then takes its 32
+// features as scalar operands, one multiply and one add per channel, and a row
+// without one is skipped by a scalar branch.  So the VALU does the valid pairs'
+// operations only (k_conv_generic multiplies zeros for the absent rows of its
+// 16- or 32-row blocks, and its LDS reads take longer than its arithmetic).
+// Sums in the reference's order: bias, then per valid offset in k order a
+// partial sum over the input channels, mul and add rounded separately.
+// Needs Ci % 32 == 0 and Co % 4 == 0 (whole 16-byte pieces of a weight row).
+// ---------------------------------------------------------------------------
+template <int R, int NW>
+__global__ void __launch_bounds__(64 * NW) k_conv_rows_f32(const float * __restrict__ x,
+                                                           const int32_t * __restrict__ table,
+                                                           const float * __restrict__ w32,
+                                                           const float * __restrict__ bias, float * __restrict__ y,
+                                                           int64_t n, int ci, int co) {
+#pragma clang fp contract(off)
+    constexpr int CH = 32, SLOTS = 3, SLOT = CH * 64;  // floats per slot
+    constexpr int PER = 8 / NW;                        // 1 KB loads per wavefront and chunk
+    static_assert(PER >= 1 && 8 % NW == 0, "a chunk is eight loads");
+    __shared__ __attribute__((aligned(1024))) float s_w[SLOTS * SLOT];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row0 = ((int64_t) blockIdx.x * NW + wave) * R;
+    const int col0 = blockIdx.y * 64, col = col0 + lane;
+    const bool ok = col < co;
+    const int chunks = ci / CH;
+    const int steps = 27 * chunks;
+    float acc[R], part[R];
+    const float b = ok && bias != nullptr ? bias[col] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = b;
+    // Weight load j: input channels 4 j' .. 4 j' + 3 of the chunk (j' = wave *
+    // PER + j), 16 pieces of 4 output channels each; pieces past the last
+    // channel read the next row or, past the buffer, zeros, and no lane that
+    // stores uses them.
+    const __amdgpu_buffer_rsrc_t wres =
+        __builtin_amdgcn_make_buffer_rsrc((void *) w32, 0, (int) (108ll * ci * co), 0x00020000);
+    const uint32_t ring = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) float *) s_w;
+    uint32_t wv[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+        wv[j] = (uint32_t) ((((wave * PER + j) * 4 + (lane >> 4)) * co + col0 + (lane & 15) * 4) * 4);
+    auto fetch = [&](int step) {
+        const uint32_t slot = ring + (uint32_t) (step % SLOTS * SLOT * 4);
+        const int s = step < steps ? step : steps - 1;
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            dma_b128(wres, slot + (uint32_t) (wave * PER + j) * 1024u, wv[j], (uint32_t) s * (uint32_t) (CH * 4) * (uint32_t) co);
+    };
+    int32_t src[R];
+    auto sources = [&](int k) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            src[r] = row0 + r < n ? __builtin_amdgcn_readfirstlane(table[(row0 + r) * kMapRow + k]) : -1;
+            part[r] = 0.0f;
+        }
+    };
+    int k = 0, chunk = 0;
+    sources(0);
+    fetch(0);
+    fetch(1);
+    for (int step = 0; step < steps; ++step) {
+        wait_vmcnt<PER>();
+        lds_barrier();  // the step's weights are there, and the slot of step - 1 is free
+        fetch(step + 2);
+        float wc[CH];
+        const float * ws = s_w + step % SLOTS * SLOT + lane;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) wc[j] = ws[j * 64];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (src[r] < 0) continue;
+            const float * xr = x + (int64_t) src[r] * ci + chunk * CH;
+            float s = part[r];
+#pragma unroll
+            for (int j = 0; j < CH; ++j) s = s + xr[j] * wc[j];
+            part[r] = s;
+        }
+        if (++chunk == chunks) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (src[r] >= 0) acc[r] = acc[r] + part[r];
+            }
+            chunk = 0;
+            if (++k < 27) sources(k);
+        }
+    }
+    wait_vmcnt<0>();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (ok && row0 + r < n) y[(row0 + r) * co + col] = acc[r];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // MFMA kernel (bf16 / fp16 storage).
 // ---------------------------------------------------------------------------
 // WR wavefronts split the rows (32 each), 4/WR the BN channels: WR = 2 for
@@ -1229,10 +1329,29 @@ __global__ void __launch_bounds__(64 * NW, NW * AP == 8 ? 1 : 2) k_conv_mfma_wre
 
 hipError_t launch_conv_generic(int dtype, const void * x, const int32_t * nbr, const float * w32, const float * bias,
                                void * y, int64_t n, int ci, int co, hipStream_t s) {
+    if (dtype == kF32 && ci % 32 == 0 && co % 4 == 0 && 108ll * ci * co <= (int64_t) INT32_MAX) {
+        // Rows per wavefront: more of them share a wavefront's weight reads,
+        // fewer give the GPU more wavefronts.  Measured (ms, R = 1 / 2 / 4 /
+        // 8, k_conv_generic last): 1,500 rows 64 -> 64 0.026 / 0.035 / 0.055 /
+        // 0.094, 0.096; 5,000 rows 32 -> 64 0.023 / 0.026 / 0.032 / 0.054,
+        // 0.055; 14,648 rows 64 -> 64 (config 1) 0.111 / 0.100 / 0.088 /
+        // 0.161, 0.160; 100,000 rows 128 -> 128 2.37 / 1.97 / 1.68 / 1.59,
+        // 2.28.
+        const int64_t col_blocks = (co + 63) / 64, parts = n * col_blocks;
+#define TSH_ROWS(RV)                                                                                         \
+    k_conv_rows_f32<RV, 4><<<dim3((unsigned) ((n + 4 * RV - 1) / (4 * RV)), (unsigned) col_blocks), 256, 0, s>>>( \
+        (const float *) x, nbr, w32, bias, (float *) y, n, ci, co)
+        if (parts < 7000) TSH_ROWS(1);
+        else if (parts < 11000) TSH_ROWS(2);
+        else if (parts < 60000) TSH_ROWS(4);
+        else TSH_ROWS(8);
+#undef TSH_ROWS
+        return hipGetLastError();
+    }
     // Two rows per lane, or one (twice the blocks) when the whole conv is
     // fewer than 1024 tiles of 32 rows x 32 input channels x 64 outputs: the
-    // GPU then runs short of blocks (config 1, 64 -> 64: 0.192 -> 0.169 ms;
-    // larger convs measured slower with one row per lane).
+    // GPU then runs short of blocks (larger convs measured slower with one row
+    // per lane).
     const int64_t tiles32 = (n + 31) / 32 * ((co + 63) / 64) * ((ci + 31) / 32);
     const int tm = tiles32 < 1024 ? 1 : 2;
     const dim3 grid((unsigned) ((n + 16 * tm - 1) / (16 * tm)), (unsigned) ((co + 63) / 64));
