@@ -11,6 +11,8 @@
 // backends (trellis_sparse_vulkan.c:163-187); separate instances are
 // independent.  Every call enqueues on the instance's own stream; calls that
 // hand data back to the host (download_*, build_c2s_map*, n_out) synchronise.
+#include <sys/mman.h>
+
 #include <algorithm>
 #include <chrono>
 #include <cstdio>
@@ -105,6 +107,10 @@ struct Backend {
     // and the event the host spins on for them (allocated at creation).
     int32_t * host_words = nullptr;
     hipEvent_t words_ready = nullptr;
+    // Stream and event for a download that overlaps the backend stream's later
+    // work (the mesh vertices; created on first use).
+    hipStream_t copy_stream = nullptr;
+    hipEvent_t copy_from = nullptr;
     // Timing.
     bool profiling = false;
     std::vector<StageMark> pending;
@@ -269,6 +275,17 @@ void parallel_copy(void * dst, const void * src, size_t bytes) {
     }
     memcpy(dst, src, chunk);
     for (auto & th : pool) th.join();
+}
+
+// Memory for an array that the caller will free(): large arrays on 2 MiB
+// boundaries with huge pages asked for, since filling fresh 4 KiB pages costs
+// more in page faults than in copying.
+void * host_array(size_t bytes) {
+    constexpr size_t kHuge = (size_t) 2 << 20;
+    if (bytes < 2 * kHuge) return malloc(bytes);
+    void * p = aligned_alloc(kHuge, (bytes + kHuge - 1) / kHuge * kHuge);
+    if (p != nullptr) (void) madvise(p, bytes / kHuge * kHuge, MADV_HUGEPAGE);  // a hint: its failure is none
+    return p;
 }
 
 // Pinned staging of at least `bytes` (the stream has no transfer pending on
@@ -1705,19 +1722,75 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
     if (r == nullptr) st = TRELLIS_STATUS_OUT_OF_MEMORY;
     if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, 16, &flags);
     int32_t hf[4] = {0, 0, 0, 0}, dup[2] = {0, 0};
+    const size_t vbytes = (size_t) n * 12;
+    float * hv = nullptr;
+    int32_t * hfaces = nullptr;
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, vbytes, &vert);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 4, &wgt);
+    if (st == TRELLIS_STATUS_OK) st = pinned_reserve(be, vbytes);
+    if (st == TRELLIS_STATUS_OK) {
+        hv = (float *) host_array(vbytes);
+        if (hv == nullptr) st = fail(be, TRELLIS_STATUS_OUT_OF_MEMORY, "host allocation");
+    }
+    if (st == TRELLIS_STATUS_OK && be->copy_stream == nullptr) {
+        hipError_t err = hipEventCreateWithFlags(&be->copy_from, hipEventDisableTiming);
+        if (err == hipSuccess) err = hipStreamCreateWithFlags(&be->copy_stream, hipStreamNonBlocking);
+        if (err != hipSuccess && be->copy_from != nullptr) {
+            (void) hipEventDestroy(be->copy_from);
+            be->copy_from = nullptr;
+        }
+        st = hip_status(be, err, "flex_dual_grid_mesh copy stream");
+    }
+    // Check and vertices first: the vertices travel to pinned memory on the
+    // copy stream while the backend stream builds the corner map and counts
+    // the quads.
+    bool copying = false;
     if (st == TRELLIS_STATUS_OK) {
         stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
         hipError_t err = launch_fill_i32((int32_t *) flags.ptr, 4, 0, s);
         if (err == hipSuccess) {
             err = launch_fdg_check(dt, coords, feats->ptr, n, channels, resolution, (int32_t *) flags.ptr, s);
         }
+        if (err == hipSuccess) {
+            err = launch_fdg_vertices(dt, coords, feats->ptr, n, channels, resolution, (float *) vert.ptr,
+                                      (float *) wgt.ptr, s);
+        }
         stage_end(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
-        st = hip_status(be, err, "flex_dual_grid_mesh check");
+        if (err == hipSuccess) err = hipEventRecord(be->copy_from, s);
+        if (err == hipSuccess) err = hipStreamWaitEvent(be->copy_stream, be->copy_from, 0);
+        if (err == hipSuccess) {
+            err = hipMemcpyAsync(be->pinned, vert.ptr, vbytes, hipMemcpyDeviceToHost, be->copy_stream);
+            copying = err == hipSuccess;
+        }
+        st = hip_status(be, err, "flex_dual_grid_mesh vertices");
     }
     if (st == TRELLIS_STATUS_OK) st = rulebook_build_device(be, coords, n, r);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 4, &counts);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 4, &first);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, 16, &total);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, scan_tmp_bytes(n), &tmp);
     if (st == TRELLIS_STATUS_OK) {
-        hipError_t err = hipMemcpyAsync(hf, flags.ptr, 16, hipMemcpyDeviceToHost, s);
-        if (err == hipSuccess) err = hipMemcpyAsync(dup, r->counters.ptr, 8, hipMemcpyDeviceToHost, s);
+        stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
+        hipError_t err = launch_fdg_count(dt, feats->ptr, (const int32_t *) r->rows.ptr, n, channels,
+                                          (int32_t *) counts.ptr, s);
+        if (err == hipSuccess) {
+            err = launch_scan_exclusive((const int32_t *) counts.ptr, (int32_t *) first.ptr, n, (int32_t *) total.ptr,
+                                        tmp.ptr, s);
+        }
+        stage_end(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
+        st = hip_status(be, err, "flex_dual_grid_mesh count");
+    }
+    // The copy is waited for on every path: the pinned buffer and the vertex
+    // block are reused after this call.
+    if (copying) {
+        const hipError_t err = hipStreamSynchronize(be->copy_stream);
+        if (st == TRELLIS_STATUS_OK) st = hip_status(be, err, "flex_dual_grid_mesh download");
+        if (st == TRELLIS_STATUS_OK) parallel_copy(hv, be->pinned, vbytes);
+    }
+    int32_t quads = 0;
+    if (st == TRELLIS_STATUS_OK) {
+        hipError_t err = hipMemcpyAsync(dup, r->counters.ptr, 8, hipMemcpyDeviceToHost, s);
+        if (err == hipSuccess) err = read_words(be, s, hf, flags.ptr, 4, &quads, total.ptr, 1);
         if (err == hipSuccess) err = hipStreamSynchronize(s);
         st = hip_status(be, err, "flex_dual_grid_mesh flags");
     }
@@ -1728,29 +1801,9 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
     if (st == TRELLIS_STATUS_OK && dup[1] != 0) {
         st = fail(be, TRELLIS_STATUS_PARSE_ERROR, "flex_dual_grid_mesh: repeated coordinate");
     }
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 12, &vert);
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 4, &wgt);
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 4, &counts);
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 4, &first);
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, 16, &total);
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, scan_tmp_bytes(n), &tmp);
-    int32_t quads = 0;
-    if (st == TRELLIS_STATUS_OK) {
-        stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
-        const int32_t * nbr = (const int32_t *) r->rows.ptr;
-        hipError_t err = launch_fdg_vertices(dt, coords, feats->ptr, n, channels, resolution, (float *) vert.ptr,
-                                             (float *) wgt.ptr, s);
-        if (err == hipSuccess) err = launch_fdg_count(dt, feats->ptr, nbr, n, channels, (int32_t *) counts.ptr, s);
-        if (err == hipSuccess) {
-            err = launch_scan_exclusive((const int32_t *) counts.ptr, (int32_t *) first.ptr, n, (int32_t *) total.ptr,
-                                        tmp.ptr, s);
-        }
-        stage_end(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
-        if (err == hipSuccess) err = read_words(be, s, &quads, total.ptr, 1);
-        st = hip_status(be, err, "flex_dual_grid_mesh count");
-    }
+    const size_t fbytes = (size_t) quads * 24;
     if (st == TRELLIS_STATUS_OK && quads > 0) {
-        st = dev_alloc(be, (size_t) quads * 24, &faces);
+        st = dev_alloc(be, fbytes, &faces);
         if (st == TRELLIS_STATUS_OK) {
             stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
             st = hip_status(be,
@@ -1759,33 +1812,16 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
                             "flex_dual_grid_mesh faces");
             stage_end(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
         }
-    }
-    float * hv = nullptr;
-    int32_t * hfaces = nullptr;
-    if (st == TRELLIS_STATUS_OK) {
-        hv = (float *) malloc((size_t) n * 12);
-        hfaces = quads > 0 ? (int32_t *) malloc((size_t) quads * 24) : nullptr;
-        if (hv == nullptr || (quads > 0 && hfaces == nullptr)) {
-            st = TRELLIS_STATUS_OUT_OF_MEMORY;
-        } else {
-            // Both arrays through the pinned staging buffer (full-rate
-            // transfers), then copied into the caller's malloc-owned arrays.
-            const size_t vbytes = (size_t) n * 12, voff = (vbytes + 255) / 256 * 256;
-            const size_t fbytes = (size_t) quads * 24;
-            st = pinned_reserve(be, voff + fbytes);
-            if (st == TRELLIS_STATUS_OK) {
-                char * stage = (char *) be->pinned;
-                hipError_t err = hipMemcpyAsync(stage, vert.ptr, vbytes, hipMemcpyDeviceToHost, s);
-                if (err == hipSuccess && quads > 0) {
-                    err = hipMemcpyAsync(stage + voff, faces.ptr, fbytes, hipMemcpyDeviceToHost, s);
-                }
-                if (err == hipSuccess) err = hipStreamSynchronize(s);
-                st = hip_status(be, err, "flex_dual_grid_mesh download");
-                if (st == TRELLIS_STATUS_OK) {
-                    parallel_copy(hv, stage, vbytes);
-                    if (quads > 0) parallel_copy(hfaces, stage + voff, fbytes);
-                }
-            }
+        if (st == TRELLIS_STATUS_OK) st = pinned_reserve(be, fbytes);
+        if (st == TRELLIS_STATUS_OK) {
+            hfaces = (int32_t *) host_array(fbytes);
+            if (hfaces == nullptr) st = fail(be, TRELLIS_STATUS_OUT_OF_MEMORY, "host allocation");
+        }
+        if (st == TRELLIS_STATUS_OK) {
+            hipError_t err = hipMemcpyAsync(be->pinned, faces.ptr, fbytes, hipMemcpyDeviceToHost, s);
+            if (err == hipSuccess) err = hipStreamSynchronize(s);
+            st = hip_status(be, err, "flex_dual_grid_mesh download");
+            if (st == TRELLIS_STATUS_OK) parallel_copy(hfaces, be->pinned, fbytes);
         }
     }
     for (DevMem * d : {&cd, &flags, &vert, &wgt, &counts, &first, &total, &tmp, &faces}) dev_release(be, d);
@@ -1902,6 +1938,8 @@ void op_destroy(trellis_sparse_backend * backend) {
     if (be->pinned != nullptr) (void) hipHostFree(be->pinned);
     if (be->host_words != nullptr) (void) hipHostFree(be->host_words);
     if (be->words_ready != nullptr) (void) hipEventDestroy(be->words_ready);
+    if (be->copy_from != nullptr) (void) hipEventDestroy(be->copy_from);
+    if (be->copy_stream != nullptr) (void) hipStreamDestroy(be->copy_stream);
     (void) hipStreamDestroy(be->stream);
     delete be;
 }
