@@ -445,7 +445,8 @@ trellis_status trellis_sparse_hip_dump_map_coords(trellis_sparse_hip_dump * dump
  * gamma and beta may be NULL).
  *   c = 64, 128, 256: one kernel; each intermediate is rounded to the storage
  * type where the slot sequence stores it, and the 4c-wide hidden rows never
- * leave the chip.
+ * leave the chip.  At c = 256 on few rows the same steps and roundings run as
+ * row_norm and two GEMM kernels through n x c and n x 4c intermediates.
  *   c a multiple of 128 from 512 (the decoder's 512 and 1024 levels, where a
  * 128-row tile's normalised rows alone would take 128 KB of the 160 KB of
  * LDS): row_norm, then mlp0 + SiLU and mlp2 as GEMMs through n x c and

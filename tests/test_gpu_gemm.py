@@ -42,3 +42,41 @@ def test_linear_vs_oracle(backends, n, ci, co, silu):
     exp = sh.storage_round(orc.linear(x[rows], w, b, rows.size, ci, co, silu=silu), dtype)
     e = np.max(np.abs(got[rows] - exp) / np.maximum(1.0, np.abs(exp)))
     assert e <= TOL[dtype]
+
+
+@pytest.mark.parametrize("n", [1, 257, 12000, 12001])
+def test_convnext_tail_256_vs_oracle(backends, n):
+    """The ConvNeXt tail at C = 256 on both sides of the row count where the fused kernel takes over from row_norm and two
+    GEMMs, and below it on the fused kernel too, which runs where the intermediates cannot be allocated (their allocation
+    is made to fail) and where eps = 0.  Rounded where the slots store, the two routes differ by the order of fp32 sums: an
+    intermediate one unit apart here and there (of 256 or 1,024 summed), then the last roundings of the second linear and
+    the add, 2^-7 each in bf16 and 2^-10 in fp16; 2^-8 (2^-11) more for the intermediates."""
+    c = 256
+    dtype = sh.F16 if n % 2 else sh.BF16
+    tol = 2.5 * TOL[dtype]
+    be = backends[dtype]
+    rng = np.random.default_rng(n)
+    rnd = lambda a: sh.storage_round(a, dtype)
+    x, res = rnd(rng.standard_normal((n, c))), rnd(rng.standard_normal((n, c)))
+    gamma, beta = (1 + 0.1 * rng.standard_normal(c)).astype(np.float32), np.zeros(c, np.float32)
+    w0, w2 = rnd(rng.standard_normal((4 * c, c)) / 16), rnd(rng.standard_normal((c, 4 * c)) / 32)
+    b0, b2 = (0.1 * rng.standard_normal(4 * c)).astype(np.float32), (0.1 * rng.standard_normal(c)).astype(np.float32)
+    rows = np.unique(np.concatenate([np.arange(min(n, 140)), np.arange(max(0, n - 140), n)]))
+    e = rnd(orc.row_norm(x[rows], gamma, beta, rows.size, c, 1e-6))
+    e = rnd(orc.linear(e, w0, b0, rows.size, c, 4 * c, silu=True))
+    e = rnd(orc.add(res[rows], rnd(orc.linear(e, w2, b2, rows.size, 4 * c, c))))
+    xb, rb, yb = be.upload(x), be.upload(res), be.alloc(n * c)
+
+    def check(eps, allocs=-1):
+        be.fail_alloc(allocs)
+        try:
+            be.convnext_mlp(xb, gamma, beta, w0, b0, w2, b2, rb, yb, n, c, eps)
+        finally:
+            be.fail_alloc(-1)
+        got = be.download(yb).reshape(n, c)[rows]
+        assert np.max(np.abs(got - e) / np.maximum(1.0, np.abs(e))) <= tol
+
+    check(1e-6)
+    check(0.0)  # the rows' variances are near 1: the same result
+    be.trim(sh.TRIM_FREE_BUFFERS)
+    check(1e-6, allocs=0)

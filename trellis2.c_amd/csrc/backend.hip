@@ -664,7 +664,8 @@ void op_free_buffer(trellis_sparse_backend * backend, trellis_sparse_buffer * bu
 // forms the sum.
 trellis_status linear_impl(trellis_sparse_backend * backend, const trellis_sparse_buffer * x, const float * weight,
                            const float * bias, trellis_sparse_buffer * y, int64_t n, int ci, int co, int silu,
-                           const trellis_sparse_buffer * residual = nullptr, trellis_sparse_buffer * scratch = nullptr) {
+                           const trellis_sparse_buffer * residual = nullptr, trellis_sparse_buffer * scratch = nullptr,
+                           bool library = true) {
     if (backend == nullptr) return TRELLIS_STATUS_INVALID_ARGUMENT;
     Backend * be = as_backend(backend);
     if (weight == nullptr || n <= 0 || ci <= 0 || co <= 0 || !float_buffer_ok(be, x, (size_t) n * ci) ||
@@ -687,7 +688,7 @@ trellis_status linear_impl(trellis_sparse_backend * backend, const trellis_spars
     // Wide shapes: the platform GEMM library when it has a plan (workspace
     // from the pool on first use; without it, or without a plan, the kernels
     // below run).
-    if (be->policy.linear_algo == TRELLIS_SPARSE_HIP_LINEAR_AUTO && linear_lt_wanted(dt, n, ci, co)) {
+    if (library && be->policy.linear_algo == TRELLIS_SPARSE_HIP_LINEAR_AUTO && linear_lt_wanted(dt, n, ci, co)) {
         constexpr size_t kLtWorkspace = size_t(32) << 20;
         if (be->lt == nullptr) be->lt = linear_lt_create();
         if (be->lt_ws.ptr == nullptr && dev_alloc(be, kLtWorkspace, &be->lt_ws) != TRELLIS_STATUS_OK) {
@@ -760,20 +761,21 @@ bool mlp_composed_supported(int dtype, int c) { return (dtype == kF16 || dtype =
 trellis_status mlp_composed(trellis_sparse_backend * backend, const trellis_sparse_buffer * x, const float * gamma,
                             const float * beta, const float * w0, const float * b0, const float * w2,
                             const float * b2, const trellis_sparse_buffer * residual, trellis_sparse_buffer * y,
-                            int64_t n, int c, float eps) {
+                            int64_t n, int c, float eps, bool library = true) {
     trellis_sparse_buffer *xn = nullptr, *hid = nullptr;
     trellis_status st = op_alloc_f32(backend, (size_t) n * c, &xn);
     if (st == TRELLIS_STATUS_OK) st = op_alloc_f32(backend, (size_t) n * 4 * c, &hid);
     if (st == TRELLIS_STATUS_OK) st = norm_impl(backend, x, gamma, beta, xn, n, c, eps, 0);
-    if (st == TRELLIS_STATUS_OK) st = linear_impl(backend, xn, w0, b0, hid, n, c, 4 * c, 1);
-    if (st == TRELLIS_STATUS_OK) st = linear_impl(backend, hid, w2, b2, y, n, 4 * c, c, 0, residual, xn);
+    if (st == TRELLIS_STATUS_OK) st = linear_impl(backend, xn, w0, b0, hid, n, c, 4 * c, 1, nullptr, nullptr, library);
+    if (st == TRELLIS_STATUS_OK) st = linear_impl(backend, hid, w2, b2, y, n, 4 * c, c, 0, residual, xn, library);
     if (hid != nullptr) op_free_buffer(backend, hid);
     if (xn != nullptr) op_free_buffer(backend, xn);
     return st;
 }
 
 // The ConvNeXt block's MLP tail: y = residual + W2 SiLU(W0 LN(x) + b0) + b2,
-// in one kernel for c = 64, 128 and 256, composed for wider rows.
+// in one kernel for c = 64, 128 and 256 (there from some 10,000 rows),
+// composed otherwise.
 trellis_status mlp_impl(trellis_sparse_backend * backend, const trellis_sparse_buffer * x, const float * gamma,
                         const float * beta, const float * w0, const float * b0, const float * w2, const float * b2,
                         const trellis_sparse_buffer * residual, trellis_sparse_buffer * y, int64_t n, int c,
@@ -791,6 +793,18 @@ trellis_status mlp_impl(trellis_sparse_backend * backend, const trellis_sparse_b
         }
         return fail(be, TRELLIS_STATUS_NOT_IMPLEMENTED,
                     "convnext_mlp: needs bf16/fp16 storage and c = 64, 128, 256 or a multiple of 128 from 512");
+    }
+    // C = 256 on few rows: the fused kernel's 128-row blocks leave most CUs
+    // idle and each still walks the whole hidden layer (0.040 ms from 1,000 to
+    // 10,000 rows); composed on the GEMM kernel, with the same roundings, 0.021
+    // ms on 1,000 rows, 0.028 on 5,003, 0.036 on 10,000, 0.054 (fused 0.046)
+    // on 20,000.  The fused kernel needs no intermediates and takes over where
+    // they do not fit; row_norm refuses eps = 0.
+    constexpr int64_t kComposed256Rows = 12000;
+    if (c == 256 && n <= kComposed256Rows && eps > 0.0f) {
+        const trellis_status st =
+            mlp_composed(backend, x, gamma, beta, w0, b0, w2, b2, residual, y, n, c, eps, false);
+        if (st != TRELLIS_STATUS_OUT_OF_MEMORY) return st;
     }
     CallScope scope(be);
     const void *g = nullptr, *bt = nullptr, *pw0 = nullptr, *pb0 = nullptr, *pw2 = nullptr, *pb2 = nullptr;
