@@ -65,7 +65,8 @@ def test_block_edges(backends, n, ci, co):
 
 # Row counts that take each block shape at 256 and 128 channels (64 x 64 up to 256 x 256), sampled rows.
 @pytest.mark.parametrize("ci,co,n", [(64, 256, 3000), (64, 256, 9000), (64, 256, 14648), (64, 512, 14648),
-                                     (64, 1024, 9000), (64, 1024, 14648), (64, 128, 3000), (128, 128, 14648)])
+                                     (64, 1024, 6000), (64, 1024, 8100), (64, 1024, 9000), (64, 1024, 12000),
+                                     (64, 1024, 14000), (64, 1024, 14648), (64, 128, 3000), (128, 128, 14648)])
 def test_block_shapes(backends, ci, co, n):
     dtype = sh.BF16
     rng = np.random.default_rng(n + ci + co)

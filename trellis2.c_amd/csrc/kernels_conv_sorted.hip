@@ -22,7 +22,7 @@ namespace {
 // reads past the buffer's end, which the hardware answers with zeros.  The
 // loads run SLOTS steps ahead of their MFMAs.  Plain blocks read a step's
 // fragments from LDS one step ahead, so its MFMAs wait for nothing but the
-// one barrier.  Ping-pong blocks (PP: 256 x 256, one per CU) let wavefronts
+// one barrier.  Ping-pong blocks (PP: 224 or 256 x 256, one per CU) let wavefronts
 // 0-3 (one per SIMD) and 4-7 take turns, half a step apart: one half reads
 // fragments and issues loads while the other half multiplies (256 -> 256 on
 // 300,000 rows: 0.74 -> 0.61 ms, MFMAs alone 0.46, loads and LDS alone 0.48).
@@ -35,25 +35,26 @@ namespace {
 //
 // What bounds it: the gathers and weights arrive at 20-24 B per clock and CU
 // (L2 misses to the last-level cache; 45 when all rows hit the L2), the MFMAs
-// run at 50-55 % of peak in 256 x 256 blocks, 35-40 % in 128-channel ones.
+// run at 50-55 % of peak in 224 x 256 and 256 x 256 blocks, 35-40 % in 128-channel ones.
 // Measured against the compacted schedule (ms, conv alone): 128 -> 128 on
 // 419,341 rows 0.60 -> 0.31; 256 -> 1024 on 350,000 5.1 -> 2.7; 512 -> 512 on
-// 79,523 1.11 -> 0.70; 1024 -> 1024 on 18,216 1.12 -> 0.86; 256 -> 256 on
+// 79,523 1.11 -> 0.71; 1024 -> 1024 on 18,216 1.12 -> 0.77; 256 -> 256 on
 // 5,003 0.100 -> 0.035; 64 -> 64 on 3,788,747 1.11 -> 0.85; 256 -> 128 on
 // 1,259,866 random children 1.71 -> 1.56.
 template <int DT, int BM, int BN, int RW, int CW, int SLOTS, bool PP = false>
 __global__ void __launch_bounds__(64 * RW * CW, RW * CW == 8 ? 2 : 1)
     k_conv_sorted(const typename Store<DT>::T * __restrict__ x, const int32_t * __restrict__ table,
-                  const int32_t * __restrict__ perm, const typename Store<DT>::T * __restrict__ w16, const float * __restrict__ bias,
+                  const int32_t * __restrict__ perm, const typename Store<DT>::T * __restrict__ w16,
+                  const float * __restrict__ bias,
                   typename Store<DT>::T * __restrict__ y, int64_t n, int ci, int co, int group, ConvEpilogue epi) {
     using T = typename Store<DT>::T;
     using V = typename Mfma<DT>::V;
     constexpr int NW = RW * CW, NTHR = 64 * NW;
     constexpr int QB = BM / RW / 16;   // row blocks per wavefront
     constexpr int NT = BN / CW / 16;   // column tiles per wavefront
-    constexpr int NA = BM / 16 / NW;   // A loads per wavefront and step (16 rows each)
     using R = RingShape<BM, BN, RW, CW>;
-    constexpr int WL = R::WL, NB = R::NB, SLOT = R::SLOT;  // weight loads of a step: the block's, a wavefront's
+    // Loads of a step, the block's and a wavefront's: of A, of the weights.
+    constexpr int AL = R::AL, NA = R::NA, WL = R::WL, NB = R::NB, SLOT = R::SLOT;
     constexpr int OUT = BM * BN * 2;
     constexpr int RING = SLOTS * SLOT > OUT ? SLOTS * SLOT : OUT;
     __shared__ __attribute__((aligned(1024))) unsigned char s_ring[RING];
@@ -121,8 +122,8 @@ __global__ void __launch_bounds__(64 * RW * CW, RW * CW == 8 ? 2 : 1)
     const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc((void *) w16, 0, (int) wbytes, 0x00020000);
     const uint32_t ring = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) unsigned char *) s_ring;
     constexpr uint32_t kAbsent = 0x80000000u;
-    // A load j: row block wave * NA + j, row lane / 4 of it, chunk place lane % 4.
-    const int arow = wave * NA * 16 + (lane >> 2);
+    // A load j: row block (wave * NA + j) % AL, row lane / 4 of it, chunk place lane % 4.
+    auto ablock = [&](int j) { return (wave * NA + j) % AL; };
     const uint32_t achunk = (uint32_t) (((lane & 3) ^ (((lane >> 5) & 1) << 1)) * 16);
     uint32_t av[NA];
     int32_t nsrc[NA];
@@ -138,7 +139,7 @@ __global__ void __launch_bounds__(64 * RW * CW, RW * CW == 8 ? 2 : 1)
         // Sources at the next offset (read a whole offset before their use).
         const int k = left != 0 ? __builtin_ctz(left) : 0;
 #pragma unroll
-        for (int j = 0; j < NA; ++j) nsrc[j] = s_nbr[(arow + j * 16) * kMapRow + k];
+        for (int j = 0; j < NA; ++j) nsrc[j] = s_nbr[(ablock(j) * 16 + (lane >> 2)) * kMapRow + k];
     };
     auto next_offset = [&]() {
         const bool end = left == 0;
@@ -152,7 +153,7 @@ __global__ void __launch_bounds__(64 * RW * CW, RW * CW == 8 ? 2 : 1)
     uint32_t islot = ring;
     auto load = [&](int j) {
         if (j < NA) {
-            dma_b128(xres, islot + (uint32_t) (wave * NA + j) * 1024u, av[j], (uint32_t) is * 64u);
+            dma_b128(xres, islot + (uint32_t) ablock(j) * 1024u, av[j], (uint32_t) is * 64u);
         } else {
             dma_b128(wres, islot + (uint32_t) (BM * 64 + (wave * NB + j - NA) % WL * 1024), wv[j - NA],
                      (uint32_t) ((ik * ci8 + is * 4) * co) * 16u);
@@ -293,23 +294,31 @@ hipError_t launch_t(const void * x, const int32_t * rows, const int32_t * perm, 
 // Block shapes, largest first.  cost[b - 1]: time of one round with b blocks
 // on every CU, as a fraction of a 256 x 256 block's (0.118 ms at 256 -> 256
 // with all 27 offsets); blocks per CU follow from the LDS.  Measured on 128 ..
-// 1024 channels and 2,000 .. 300,000 rows.
+// 1024 channels and 2,000 .. 350,000 rows.
 struct Shape {
     int id, bm, bn, per_cu;
     double cost[4];
 };
 constexpr Shape kShapes[] = {
     {0, 256, 256, 1, {1.0}},
-    {1, 128, 256, 1, {0.66}},
-    {2, 128, 128, 2, {0.44, 0.75}},
-    {3, 64, 128, 2, {0.33, 0.46}},
-    {4, 64, 64, 4, {0.24, 0.34, 0.50, 0.66}},
+    {1, 224, 256, 1, {0.89}},
+    {2, 192, 256, 1, {0.83}},
+    {3, 160, 256, 1, {0.77}},
+    {4, 128, 256, 1, {0.66}},
+    {5, 96, 256, 1, {0.58}},
+    {6, 128, 128, 2, {0.44, 0.75}},
+    {7, 64, 128, 2, {0.33, 0.46}},
+    {8, 64, 64, 4, {0.24, 0.34, 0.50, 0.66}},
 };
 
 // The shape that finishes first: large blocks do the most MFMA work per
-// fetched byte (256 -> 256 on 300,000 rows: 0.61 ms, 0.68 with 128 x 256,
-// 0.80 with 128 x 128), small ones fill the GPU on small sets (5,003 rows:
-// 0.113, 0.076, 0.051, 0.039 and 0.035 ms down the list).
+// fetched byte (256 -> 1024 on 350,000 rows: 2.77 ms with 256 x 256, 3.11 with
+// 128 x 256), small ones fill the GPU on small sets (256 -> 256 on 5,003 rows:
+// 0.113 ms with 256 x 256, 0.076 with 128 x 256, 0.035 with 64 x 64), and
+// between these the row count decides which fills its last round (1024 -> 1024
+// on 18,216 rows: 0.93, 0.85, 0.81, 0.77 and 0.86 ms down the list; 256 -> 256
+// on 80,000: 0.253, 0.234, 0.205, 0.193 and 0.213; on 20,000: 0.122, 0.116,
+// 0.109, 0.095, 0.081 and 0.071; on 300,000: 0.70, 0.63, 0.65, 0.67, 0.68).
 int pick_shape(int64_t n, int ci, int co, int cus, bool whole_rows) {
     // With more weights per column block than an XCD's L2 holds, blocks of few
     // columns that share a CU wait for them (512 -> 512 on 79,523 rows, 128 x
@@ -328,8 +337,10 @@ int pick_shape(int64_t n, int ci, int co, int cus, bool whole_rows) {
             const int on = (int) ((rest + cus - 1) / cus);
             t += sh.cost[on - 1] * (on > 1 ? heavy : 1.0);
         }
-        // Over many rounds blocks of unequal cost even the last one out.
-        if (rounds >= 4) t = (double) blocks / (double) cap * full;
+        // Blocks are of unequal cost (as many offsets as their rows' masks
+        // share): over more than two rounds that evens out all but a tail of
+        // about one block.
+        if (blocks > 2 * cap) t = ((double) blocks / (double) cap + 1.0) * full;
         if (best < 0 || t < best_t) {
             best = sh.id;
             best_t = t;
@@ -353,16 +364,20 @@ hipError_t launch_dt(const void * x, const int32_t * rows, const int32_t * perm,
     }
     switch (pick_shape(n, ci, co, cus, epi.mode == kEpiNorm)) {
         case 0: return TSH_SORTED(256, 256, 2, 4, 4, true);
-        case 1: return TSH_SORTED(128, 256, 2, 4, 4);
-        case 2:
+        case 1: return TSH_SORTED(224, 256, 2, 4, 4, true);
+        case 2: return TSH_SORTED(192, 256, 2, 4, 4);
+        case 3: return TSH_SORTED(160, 256, 2, 4, 4);
+        case 4: return TSH_SORTED(128, 256, 2, 4, 4);
+        case 5: return TSH_SORTED(96, 256, 2, 4, 3);
+        case 6:
             // With 8 or fewer K steps per offset a block's start and end
             // weigh more: two slots instead of four leave room for a third
             // block per CU to run under them (1,159,741 rows, 128 -> 128:
             // 0.72 -> 0.66 ms; 256 -> 128 the same either way).
             if (ci <= 128 && (n + 127) / 128 * (co / 128) >= 6 * (int64_t) cus) return TSH_SORTED(128, 128, 2, 2, 2);
             return TSH_SORTED(128, 128, 2, 2, 4);
-        case 3: return TSH_SORTED(64, 128, 2, 2, 4);
-        case 4: return TSH_SORTED(64, 64, 2, 2, 4);
+        case 7: return TSH_SORTED(64, 128, 2, 2, 4);
+        case 8: return TSH_SORTED(64, 64, 2, 2, 4);
     }
 #undef TSH_SORTED
     return hipErrorInvalidValue;

@@ -24,6 +24,7 @@ __global__ void __launch_bounds__(64 * RW * CW, 1)
     constexpr int WR = BM / RW;                 // rows per wavefront row group
     constexpr int RING = SLOTS * SLOT;
     static_assert(NT == 8, "eight adjacent channels per lane");
+    static_assert(R::AL % NW == 0, "whole loads of A");
     __shared__ __attribute__((aligned(1024))) unsigned char s_ring[RING];
 
     const int t = threadIdx.x;

@@ -14,15 +14,15 @@ template <int BM, int BN, int RW, int CW> struct RingShape {
     static constexpr int NW = RW * CW;
     static constexpr int QB = BM / RW / 16;  // row blocks per wavefront
     static constexpr int NT = BN / CW / 16;  // column tiles per wavefront
-    // Loads of 1 KB per wavefront and step: 16 rows of A each, or 64 granules
-    // of weights (with fewer of these than wavefronts some fetch the same
-    // ones, so that every wavefront counts the same number of loads).
-    static constexpr int NA = BM / 16 / NW;
+    // Loads of 1 KB per step, and per wavefront: 16 rows of A each, or 64
+    // granules of weights.  Where the wavefronts do not divide them some fetch
+    // the same ones, so that every wavefront counts the same number of loads.
+    static constexpr int AL = BM / 16;
+    static constexpr int NA = (AL + NW - 1) / NW;
     static constexpr int WL = BN / 16;
-    static constexpr int NB = WL < NW ? 1 : WL / NW;
+    static constexpr int NB = (WL + NW - 1) / NW;
     static constexpr int PER = NA + NB;
     static constexpr int SLOT = (BM + BN) * 64;
-    static_assert(NA >= 1 && BM % (16 * NW) == 0 && (WL % NW == 0 || NW % WL == 0), "whole loads");
     static_assert(QB >= 1 && NT >= 1 && BM % (16 * RW) == 0 && BN % (16 * CW) == 0, "whole MFMA tiles");
 };
 
