@@ -954,14 +954,13 @@ def main():
     hm_ms = (stages["hash"][0] + stages["map"][0]) / args.steps
     # Hash + kernel map against HBM: the work definition's bytes (hash 28 N,
     # map 16 N + 108 N + 8 P + 216, the 108 N being an [N][27] neighbour
-    # table), and the bytes the production build moves, which writes row
-    # masks and per-tile pair lists instead of that table (hash 28 N; map
-    # 16 N coordinates + 4 N masks + 5 P pairs (a 4-byte source row and a
-    # 1-byte destination row within the tile) + 2 x 108 bytes per 256-row
-    # tile of counts and list starts).
+    # table), and the bytes the production build moves (hash 28 N; map 16 N
+    # coordinates + 112 N rows of 27 neighbours and the mask + 4 N masks; where
+    # the conv takes the rows in mask order also 16 N: masks twice, 2-byte ranks
+    # out and in, places).
     hm_def_bytes = wl.hash_bytes(job.m) + wl.map_bytes(job.m, job.pairs)
-    tiles = (job.m + 255) // 256
-    hm_moved_bytes = 28.0 * job.m + 16.0 * job.m + 4.0 * job.m + 5.0 * job.pairs + 216.0 * tiles
+    algo_name = conv_schedule(spec["dtype"], job.ci, job.co, args.conv_algo)
+    hm_moved_bytes = (28.0 + 16.0 + 112.0 + 4.0 + (16.0 if algo_name == "sorted" else 0.0)) * job.m
     hm_gbs = hm_def_bytes / (hm_ms * 1e-3) / 1e9 if hm_ms > 0 else 0.0
     elem = 4 if spec["dtype"] == sh.F32 else 2
     # The conv's binding roofline: compute (2 P Ci Co at the dtype's MFMA or
@@ -976,7 +975,6 @@ def main():
         roof_achieved, roof_peak, roof_unit, roof_bound = achieved, peak_flops, "TFLOP/s", "mfma"
     # HBM bytes per conv launch come from the committed, copy-calibrated
     # rocprofv3 FETCH_SIZE / WRITE_SIZE summary for this workload and schedule.
-    algo_name = conv_schedule(spec["dtype"], job.ci, job.co, args.conv_algo)
     traffic = None
     try:
         with open(os.path.join(ROOT, "profiles", "traffic.json")) as f:
