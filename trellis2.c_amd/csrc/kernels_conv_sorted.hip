@@ -34,8 +34,10 @@ namespace {
 // measured; 125 without the swizzle).
 //
 // What bounds it: the gathers and weights arrive at 20-24 B per clock and CU
-// (L2 misses to the last-level cache; 45 when all rows hit the L2), the MFMAs
-// run at 50-55 % of peak in 224 x 256 and 256 x 256 blocks, 35-40 % in 128-channel ones.
+// (L2 misses to the last-level cache, 5.5-5.8 TB/s; 45 when all rows hit the
+// L2).  In 224 x 256 and 256 x 256 blocks the matrix cores are busy 80 % of
+// the cycles (512 -> 512 on 328,123 rows: 1.02 PFLOP/s of valid pairs, 1.49
+// with the absent ones), in 128-channel ones 36-55 %, 64-channel ones 21 %.
 // Measured against the compacted schedule (ms, conv alone): 128 -> 128 on
 // 419,341 rows 0.60 -> 0.31; 256 -> 1024 on 350,000 5.1 -> 2.7; 512 -> 512 on
 // 79,523 1.11 -> 0.71; 1024 -> 1024 on 18,216 1.12 -> 0.77; 256 -> 256 on
@@ -71,7 +73,9 @@ __global__ void __launch_bounds__(64 * RW * CW, RW * CW == 8 ? 2 : 1)
     // Blocks b, b + 8, ... run on one XCD.  With 2, 4 or 8 column blocks each
     // XCD keeps to one of them (its weights in that XCD's L2), and the row
     // blocks, whose cost rises and falls along the mask order, are dealt to
-    // the XCDs in turn.
+    // the XCDs in turn.  (A contiguous eighth of the rows per XCD, in windows
+    // of 2^15 rows, was slower: 64 -> 64 on 3,788,747 rows with its map 1.33
+    // -> 1.41 ms, 512 -> 512 on 327,689 2.73 -> 2.81.)
     const int64_t row_tiles = (n + BM - 1) / BM;
     const int col_tiles = co / BN;
     int64_t tile;
