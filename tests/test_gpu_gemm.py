@@ -1,5 +1,6 @@
-"""The linear slots' GEMM kernel (16-bit, Ci % 64 == 0, Co % 128 == 0; policy LINEAR_KERNEL) at the edges of its row
-blocks and in each block shape, plain, with SiLU, and with the residual of the composed ConvNeXt tail.
+"""The linear slots' GEMM kernel (16-bit, Ci = 64 or Ci % 128 == 0, Co % 128 == 0; policy LINEAR_KERNEL) at the edges of
+its row blocks and in each block shape, plain, with SiLU, and with the residual of the composed ConvNeXt tail; and widths
+beside it, which keep fp32 weights.
 
 Tolerance: against the oracle's linear on the same rounded inputs the fp32 sums differ by their order (some 1e-6; 1e-4
 allowed) and the rounding to the storage type by one unit in the last place where they fall on either side of a tie
@@ -42,6 +43,21 @@ def test_linear_vs_oracle(backends, n, ci, co, silu):
     exp = sh.storage_round(orc.linear(x[rows], w, b, rows.size, ci, co, silu=silu), dtype)
     e = np.max(np.abs(got[rows] - exp) / np.maximum(1.0, np.abs(exp)))
     assert e <= TOL[dtype]
+
+
+@pytest.mark.parametrize("algo", [sh.LINEAR_AUTO, sh.LINEAR_KERNEL])
+@pytest.mark.parametrize("n,ci,co", [(1, 192, 128), (300, 192, 256), (257, 320, 128), (64, 448, 384)])
+@pytest.mark.parametrize("dtype", [sh.BF16, sh.F16])
+def test_weights_between_the_mfma_widths_stay_fp32(n, ci, co, dtype, algo):
+    """Ci = 192, 320, 448: features 1, -1, 1, ... times weights 1 + 2^-12, 1, 1 + 2^-12, ... sum to ci / 2 * 2^-12, exact in
+    fp32 in any order and in both storage types; weights rounded to 8 or 11 bits would give 0.  Tolerance: none."""
+    be = sh.Backend(0, dtype, linear_algo=algo)
+    x = np.tile(np.array([1, -1], np.float32), (n, ci // 2))
+    w = np.tile(np.array([1 + 2.0 ** -12, 1], np.float32), (co, ci // 2))
+    xb, yb = be.upload(x), be.alloc(n * co)
+    be.linear(xb, w, None, yb, n, ci, co)
+    assert np.all(be.download(yb) == ci // 2 * 2.0 ** -12)
+    be.destroy()
 
 
 @pytest.mark.parametrize("n", [1, 257, 12000, 12001])

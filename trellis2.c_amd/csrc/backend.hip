@@ -679,10 +679,10 @@ trellis_status linear_impl(trellis_sparse_backend * backend, const trellis_spars
     const void * wt = nullptr;
     const void * bd = nullptr;
     const int dt = be->policy.compute_dtype;
-    // bf16/fp16 with Ci % 64 == 0 and Co % 128 == 0: the GEMM kernel; Ci = 64
-    // or Ci % 128 == 0 and other Co % 64 == 0: the MFMA linear kernel; Co <= 16
-    // (the subdivide logits): the narrow MFMA kernel; otherwise (and always
-    // for fp32) the reference-order VALU kernel.
+    // bf16/fp16 with Ci = 64 or Ci % 128 == 0: the GEMM kernel (Co % 128 == 0)
+    // or the MFMA linear kernel (other Co % 64 == 0, or rows past the GEMM's 2
+    // GiB); Co <= 16 (the subdivide logits): the narrow MFMA kernel; otherwise
+    // (and always for fp32) the reference-order VALU kernel with fp32 weights.
     trellis_status st = get_weight(be, bias, (size_t) co, kLayoutVector, 0, co, &bd);
     if (st != TRELLIS_STATUS_OK) return st;
     // Wide shapes: the platform GEMM library when it has a plan (workspace

@@ -160,8 +160,12 @@ hipError_t launch_dt(const void * x, const void * w16, const float * bias, const
 
 }  // namespace
 
+// Of the widths whose weights launch_linear_mfma rounds to the storage type too,
+// those with whole 128-column blocks: other multiples of 64 input channels
+// (192, 320, ...), which the K loop could take, keep their fp32 weights on the
+// VALU kernel.
 bool gemm_supported(int dtype, int64_t n, int ci, int co) {
-    return (dtype == kF16 || dtype == kBF16) && n > 0 && ci >= 64 && ci % 64 == 0 && co > 0 && co % 128 == 0 &&
+    return linear_mfma_supported(dtype, ci, co) && co % 128 == 0 && n > 0 &&
            n <= INT32_MAX / (2 * (int64_t) ci) && (int64_t) ci * co * 2 <= (int64_t) INT32_MAX;
 }
 

@@ -291,9 +291,11 @@ void linear_lt_destroy(LinearLt * lt);
 bool linear_lt_run(LinearLt * lt, int dtype, const void * x, const void * w16, const float * bias,
                    const void * residual, void * y, int64_t n, int ci, int co, int silu, void * workspace,
                    size_t workspace_bytes, hipStream_t s);
-// Wide linears as a GEMM through LDS (kernels_gemm.hip): 16-bit storage, Ci %
-// 64 == 0, Co % 128 == 0; the weights of launch_linear_mfma.  A non-null
-// residual (may be y) is added to the fp32 sums before the one rounding.
+// Wide linears as a GEMM through LDS (kernels_gemm.hip): 16-bit storage, Ci =
+// 64 or Ci % 128 == 0, Co % 128 == 0; weights [ci/8][co][8] in the storage
+// type, in groups of 128 columns with 8 adjacent channels per lane.  A non-null
+// residual (may be y) is added to the linear output rounded to the storage
+// type, and the sum is rounded again, as the linear and add slots do.
 bool gemm_supported(int dtype, int64_t n, int ci, int co);
 hipError_t launch_gemm(int dtype, const void * x, const void * w16, const float * bias, const void * residual,
                        void * y, int64_t n, int ci, int co, int silu, int cus, hipStream_t s);
