@@ -186,8 +186,10 @@ typedef enum trellis_sparse_hip_dtype {
  * with Ci % 64 == 0 and Co 16, 32 or a multiple of 64 an MFMA kernel over rows
  * in the order of their neighbour masks (finite weights, features up to 2
  * GiB), else COMPACT where it applies, else MASKED, else GENERIC; a schedule
- * that does not apply falls back the same way.  The choice never changes which
- * pairs contribute, only the order of fp32 summation. */
+ * that does not apply falls back the same way, and so does MASKED (to GENERIC)
+ * for weights with an infinity or NaN, which it would multiply with the zeros
+ * of missing neighbours.  The choice never changes which pairs contribute, only
+ * the order of fp32 summation. */
 typedef enum trellis_sparse_hip_conv_algo {
     TRELLIS_SPARSE_HIP_CONV_AUTO = 0,
     TRELLIS_SPARSE_HIP_CONV_GENERIC = 1,   /* one lane per output element, any channels and dtype */

@@ -1053,24 +1053,34 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
     trellis_status st = TRELLIS_STATUS_OK;
     int algo = be->policy.conv_algo;
     bool sorted = false;
+    bool finite = true;
     const void * w = nullptr;
+    // The sorted and the masked schedule multiply rows without a neighbour at
+    // an offset by zeros, so weights that are not finite, whose products would
+    // be NaN where the reference skips the offset, run one that multiplies
+    // valid pairs only: the compacted one, or the VALU one (with fp32 weights).
     if (algo == TRELLIS_SPARSE_HIP_CONV_AUTO) {
-        // The sorted schedule takes every MFMA shape with Ci % 64 == 0.  It
-        // multiplies a row without a neighbour at an offset by zeros, so
-        // weights that are not finite, whose products would be NaN where the
-        // reference skips the offset, run the compacted schedule, which
-        // multiplies valid pairs only.
+        // The sorted schedule takes every MFMA shape with Ci % 64 == 0.
         algo = TRELLIS_SPARSE_HIP_CONV_COMPACT;
         if (conv_sorted_supported(dt, ci, co, n)) {
-            st = get_weight(be, weight, wcount, kLayoutConvMfmaGrouped, ci, co, &w, &sorted);
+            st = get_weight(be, weight, wcount, kLayoutConvMfmaGrouped, ci, co, &w, &finite);
             if (st != TRELLIS_STATUS_OK) return st;
+            sorted = finite;
         }
     }
     if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT && !sorted && !conv_stream_supported(dt, ci, co)) {
         algo = TRELLIS_SPARSE_HIP_CONV_MASKED;
     }
-    if (algo == TRELLIS_SPARSE_HIP_CONV_MASKED && !conv_mfma_supported(dt, ci, co)) {
-        algo = TRELLIS_SPARSE_HIP_CONV_GENERIC;
+    if (algo == TRELLIS_SPARSE_HIP_CONV_MASKED) {
+        const bool mfma = conv_mfma_supported(dt, ci, co);
+        if (mfma && finite) {
+            st = get_weight(be, weight, wcount, kLayoutConvMfma, ci, co, &w, &finite);
+            if (st != TRELLIS_STATUS_OK) return st;
+        }
+        if (!mfma || !finite) algo = TRELLIS_SPARSE_HIP_CONV_GENERIC;
+    } else if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT && !sorted) {
+        st = get_weight(be, weight, wcount, kLayoutConvMfmaGrouped, ci, co, &w);
+        if (st != TRELLIS_STATUS_OK) return st;
     }
     const void * bd = nullptr;
     st = get_weight(be, bias, (size_t) co, kLayoutVector, 0, co, &bd);
@@ -1086,12 +1096,6 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
     }
     hipError_t err;
     if (algo == TRELLIS_SPARSE_HIP_CONV_MASKED || algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
-        if (!sorted) {
-            st = get_weight(be, weight, wcount,
-                            algo == TRELLIS_SPARSE_HIP_CONV_COMPACT ? kLayoutConvMfmaGrouped : kLayoutConvMfma, ci, co,
-                            &w);
-            if (st != TRELLIS_STATUS_OK) return st;
-        }
         if (sorted) {
             st = rulebook_ensure_order(be, rulebook);
         } else if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
