@@ -94,6 +94,33 @@ def test_repeated_coordinates(backends, ci, co):
     assert err(y, sh.storage_round(orc.Rulebook(coords).conv(x, w, None, ci, co), dtype)) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("n,ci,co", [(1, 64, 64), (700, 64, 16), (1000, 128, 32), (5000, 64, 192), (9001, 128, 128),
+                                     (14648, 64, 512)])
+def test_no_memory_for_the_order(n, ci, co):
+    """A conv on a built rulebook whose mask order cannot be allocated (every allocation fails) takes the rows in their own
+    order.  A row's sums do not depend on which rows it shares blocks with: the same bits.  Tolerance: none."""
+    dtype = sh.BF16 if n % 2 else sh.F16
+    be = sh.Backend(0, dtype)
+    rng = np.random.default_rng(n)
+    coords = np.ascontiguousarray(shell(n)[rng.permutation(n)])
+    x = rng.standard_normal((n, ci)).astype(np.float32)
+    w, b = be.keep(weights(rng, ci, co, dtype)), be.keep((0.1 * rng.standard_normal(co)).astype(np.float32))
+    xb, yb, zb = be.upload(x), be.alloc(n * co), be.alloc(n * co)
+    rb = be.build_rulebook(coords)
+    be.conv(rb, xb, w, b, yb, ci, co)
+    rb.free()
+    rb = be.build_rulebook(coords)
+    be.trim(sh.TRIM_FREE_BUFFERS)
+    be.fail_alloc(0)
+    try:
+        be.conv(rb, xb, w, b, zb, ci, co)
+    finally:
+        be.fail_alloc(-1)
+    assert np.array_equal(be.download_raw(yb), be.download_raw(zb))
+    rb.free()
+    be.destroy()
+
+
 def test_more_rows_than_a_sort_window(backends):
     """419,340 rows (the sort takes 262,144 at a time), 64 -> 128: sampled rows in every part."""
     dtype = sh.BF16

@@ -1097,7 +1097,13 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
     hipError_t err;
     if (algo == TRELLIS_SPARSE_HIP_CONV_MASKED || algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
         if (sorted) {
+            // Where the order's memory does not fit, the rows are taken in their
+            // own: the same sums, more of the multiplied rows absent.
             st = rulebook_ensure_order(be, rulebook);
+            if (st == TRELLIS_STATUS_OUT_OF_MEMORY) {
+                be->last_error.clear();
+                st = TRELLIS_STATUS_OK;
+            }
         } else if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
             st = rulebook_ensure_lists(be, rulebook);
         }
