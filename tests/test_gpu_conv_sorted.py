@@ -1,6 +1,6 @@
-"""The AUTO policy's 16-bit conv (rows in mask order) where it can go wrong: the edges of its row blocks, every block
-shape (16 to 256 channels; small sets and sets that fill the GPU), repeated coordinates, more rows than one sort
-window, and weights that are not finite.
+"""The AUTO policy's 16-bit conv (rows in their own order, and in mask order) where it can go wrong: the edges of its row
+blocks, every block shape (16 to 256 channels; small sets and sets that fill the GPU), repeated coordinates, more rows
+than one sort window, no memory for the order, and weights that are not finite.
 
 Tolerance: both sides compute on the same rounded inputs, so they differ by their fp32 summation orders (some 1e-6 to
 1e-5 here; 1e-4 allowed) and by the one rounding to the storage type.  Sums on either side of a tie round to
@@ -36,14 +36,31 @@ def weights(rng, ci, co, dtype):
     return sh.storage_round(rng.standard_normal((co, 27, ci)) / math.sqrt(27 * ci), dtype)
 
 
+ORDER_WORK = 4e9  # rows x input x output channels of the convs on a rulebook, from which they take its rows in mask order
+
+
+def reach_order(be, rb):
+    """Runs convs on a rulebook until the next one takes its rows in mask order."""
+    ci, co = (64, 64) if rb.n >= 4096 else (256, 1024)
+    xb, yb = be.upload(np.ones((rb.n, ci), np.float32)), be.alloc(rb.n * co)
+    w = be.keep(np.zeros((co, 27, ci), np.float32))
+    for _ in range(math.ceil(ORDER_WORK / (rb.n * ci * co))):
+        be.conv(rb, xb, w, None, yb, ci, co)
+    be.synchronize()
+
+
 def run(be, coords, x, w, b, ci, co):
+    """One conv on a fresh rulebook, and again with the rows in mask order: the same bits."""
     n = coords.shape[0]
     rb = be.build_rulebook(coords)
-    xb, yb = be.upload(x), be.alloc(n * co)
+    xb, yb, zb = be.upload(x), be.alloc(n * co), be.alloc(n * co)
+    w, b = be.keep(w), None if b is None else be.keep(b)
+    be.conv(rb, xb, w, b, zb, ci, co)
+    reach_order(be, rb)
     be.conv(rb, xb, w, b, yb, ci, co)
-    y = be.download(yb).reshape(n, co)
     rb.free()
-    return y
+    assert np.array_equal(be.download_raw(yb), be.download_raw(zb))
+    return be.download(yb).reshape(n, co)
 
 
 def shell(n):
@@ -106,18 +123,28 @@ def test_no_memory_for_the_order(n, ci, co):
     x = rng.standard_normal((n, ci)).astype(np.float32)
     w, b = be.keep(weights(rng, ci, co, dtype)), be.keep((0.1 * rng.standard_normal(co)).astype(np.float32))
     xb, yb, zb = be.upload(x), be.alloc(n * co), be.alloc(n * co)
-    rb = be.build_rulebook(coords)
-    be.conv(rb, xb, w, b, yb, ci, co)
-    rb.free()
-    rb = be.build_rulebook(coords)
-    be.trim(sh.TRIM_FREE_BUFFERS)
-    be.fail_alloc(0)
-    try:
-        be.conv(rb, xb, w, b, zb, ci, co)
-    finally:
-        be.fail_alloc(-1)
+    wide = be.keep(np.zeros((1024, 27, 1024), np.float32))
+    wx, wy = be.upload(np.zeros((n, 1024), np.float32)), be.alloc(n * 1024)
+    be.conv(be.build_rulebook(coords), wx, wide, None, wy, 1024, 1024)  # its weights
+    for out, starved in ((yb, False), (zb, True)):
+        rb = be.build_rulebook(coords)
+        be.profile(True)
+        be.profile_read()
+        if starved:
+            be.trim(sh.TRIM_FREE_BUFFERS)
+            be.fail_alloc(0)
+        try:
+            for _ in range(math.ceil(ORDER_WORK / (n * 1024 * 1024)) - 1):
+                be.conv(rb, wx, wide, None, wy, 1024, 1024)
+            assert be.profile_read()["map"][1] == 0  # not yet
+            be.conv(rb, wx, wide, None, wy, 1024, 1024)
+            be.conv(rb, xb, w, b, out, ci, co)
+        finally:
+            be.fail_alloc(-1)
+        assert be.profile_read()["map"][1] == (0 if starved else 1)
+        be.profile(False)
+        rb.free()
     assert np.array_equal(be.download_raw(yb), be.download_raw(zb))
-    rb.free()
     be.destroy()
 
 

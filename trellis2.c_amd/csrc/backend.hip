@@ -912,7 +912,28 @@ trellis_status rulebook_ensure_lists(Backend * be, const trellis_sparse_rulebook
     return TRELLIS_STATUS_OK;
 }
 
-// The rows' mask order, built on first use by the convs that take it.
+// The mask order costs 15 us (four launches) and 18 us more per million rows,
+// whatever the conv; what it saves a conv grows with the conv.  Sorted convs
+// therefore run in row order until their work on the rulebook (rows x input x
+// output channels, at least 64 of these) reaches kOrderWork, so that a set used
+// once or twice in a small conv pays for no order, and one that many convs
+// share soon has it.  Fresh map and one conv, in us, row order against mask
+// order: 1 row 64 -> 64 17 (25); 5,000 rows 64 -> 64 28 (44), 256 -> 256 55
+// (70); 60,000 rows 64 -> 64 44 (60), 256 -> 256 161 (168); 14,648 rows 512 ->
+// 512 182 (183), 1024 -> 1024 571 (525); 100,000 rows 128 -> 128 105 (119), 256
+// -> 256 268 (251); 419,340 rows 64 -> 64 168 (192), 128 -> 128 360 (347), 256
+// -> 256 1089 (899); 1,200,000 rows 64 -> 64 450 (427); 3,788,747 rows 64 -> 64
+// 1429 (1300).  The conv alone on an ordered set: 5,000 rows 256 -> 256 36 (row
+// order 37), 100,000 rows 256 -> 256 211 (244).  The sums are the same bits in
+// either order.
+constexpr double kOrderWork = 4e9;
+bool rulebook_order_pays(const trellis_sparse_rulebook * rc, int ci, int co) {
+    auto * r = const_cast<trellis_sparse_rulebook *>(rc);
+    r->conv_work += (double) r->n * ci * std::max(co, 64);
+    return r->conv_work >= kOrderWork;
+}
+
+// The rows' mask order.
 trellis_status rulebook_ensure_order(Backend * be, const trellis_sparse_rulebook * rc) {
     auto * r = const_cast<trellis_sparse_rulebook *>(rc);
     if (r->perm.ptr != nullptr) return TRELLIS_STATUS_OK;
@@ -1099,7 +1120,7 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
         if (sorted) {
             // Where the order's memory does not fit, the rows are taken in their
             // own: the same sums, more of the multiplied rows absent.
-            st = rulebook_ensure_order(be, rulebook);
+            if (rulebook_order_pays(rulebook, ci, co)) st = rulebook_ensure_order(be, rulebook);
             if (st == TRELLIS_STATUS_OUT_OF_MEMORY) {
                 be->last_error.clear();
                 st = TRELLIS_STATUS_OK;

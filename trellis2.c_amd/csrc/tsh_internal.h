@@ -156,8 +156,9 @@ struct trellis_sparse_rulebook {
     tsh::DevMem tile_off;    // int32  [n_tiles][27] start of (tile, k) in the pair arrays
     tsh::DevMem pair_src;    // int32  [n_tiles][kMapTile * 27]: per tile, offsets ascending, dst ascending
     tsh::DevMem pair_dst;    // uint8  [n_tiles][kMapTile * 27]: destination row within the tile
-    // Mask order (built by the first conv that takes the rows in it).
+    // Mask order (built once the sorted convs' work pays for it).
     tsh::DevMem perm;        // int32  [n] row at each place
+    double conv_work = 0.0;  // of the sorted convs so far (kOrderWork)
 };
 
 struct trellis_sparse_c2s_device_map {
