@@ -357,7 +357,15 @@ template <int DT>
 hipError_t launch_dt(const void * x, const int32_t * rows, const int32_t * perm, const void * w16, const float * bias,
                      void * y, int64_t n, int ci, int co, int cus, hipStream_t s, const ConvEpilogue & epi) {
 #define TSH_SORTED(...) launch_t<DT, __VA_ARGS__>(x, rows, perm, w16, bias, y, n, ci, co, s, epi)
-    if (co == 16) return TSH_SORTED(128, 16, 4, 1, 3);
+    // 16 and 32 channels: 128 rows of four wavefronts, four slots, three blocks
+    // per CU.  Measured on ordered rows (us, conv alone; the compacted kernel
+    // last): 64 -> 16 on 1,200,000 rows 225, with three slots (also three
+    // blocks) 230, two 235, 256 rows and two slots 254, two wavefronts 242;
+    // 252; 512 -> 16 on 5,000 rows 60, 83, 121, 148, 83; 169; on 60,000 140,
+    // 146, 167, 204, 144; 182.  128 -> 32 on 1,200,000 rows 426, three slots
+    // 433, two 453, 64 rows 459, 256 rows 470; 510; on 5,000 rows 17, 18, 24,
+    // 14, 32; 54.
+    if (co == 16) return TSH_SORTED(128, 16, 4, 1, 4);
     if (co == 32) return TSH_SORTED(128, 32, 4, 1, 4);
     if (co % 128 != 0) {
         // 64-channel blocks: 128 rows once those fill the GPU (3,788,747
