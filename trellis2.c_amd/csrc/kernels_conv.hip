@@ -1329,7 +1329,10 @@ __global__ void __launch_bounds__(64 * NW, NW * AP == 8 ? 1 : 2) k_conv_mfma_wre
 
 hipError_t launch_conv_generic(int dtype, const void * x, const int32_t * nbr, const float * w32, const float * bias,
                                void * y, int64_t n, int ci, int co, hipStream_t s) {
-    if (dtype == kF32 && ci % 32 == 0 && co % 4 == 0 && 108ll * ci * co <= (int64_t) INT32_MAX) {
+    // A single voxel has the centre offset only, which k_conv_generic alone
+    // walks (64 -> 64 0.006 ms against 0.009, 512 -> 16 0.029 against 0.047; two
+    // rows 0.013 against 0.010 and 0.081 against 0.054).
+    if (dtype == kF32 && n > 1 && ci % 32 == 0 && co % 4 == 0 && 108ll * ci * co <= (int64_t) INT32_MAX) {
         // Rows per wavefront: more of them share a wavefront's weight reads,
         // fewer give the GPU more wavefronts.  Measured (ms, R = 1 / 2 / 4 /
         // 8, k_conv_generic last): 1,500 rows 64 -> 64 0.026 / 0.035 / 0.055 /
