@@ -882,34 +882,57 @@ trellis_status op_add(trellis_sparse_backend * backend, const trellis_sparse_buf
 }
 
 // ---- rulebook -------------------------------------------------------------------
-// The pair lists of a rulebook, built on first use by the convs that walk
-// them (and the pair and statistics downloads).
+trellis_status alloc_lists(Backend * be, trellis_sparse_rulebook * r, PairLists * lists) {
+    const size_t tiles = (size_t) r->n_tiles;
+    trellis_status st = dev_alloc(be, tiles * 27 * 4, &r->tile_counts);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, tiles * 27 * 4, &r->tile_off);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, tiles * kMapTile * 27 * 4, &r->pair_src);
+    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, tiles * kMapTile * 27, &r->pair_dst);
+    if (st != TRELLIS_STATUS_OK) {
+        for (DevMem * m : {&r->tile_counts, &r->tile_off, &r->pair_src, &r->pair_dst}) dev_release(be, m);
+        return st;
+    }
+    lists->tile_counts = (int32_t *) r->tile_counts.ptr;
+    lists->tile_off = (int32_t *) r->tile_off.ptr;
+    lists->pair_src = (int32_t *) r->pair_src.ptr;
+    lists->pair_dst = (uint8_t *) r->pair_dst.ptr;
+    return TRELLIS_STATUS_OK;
+}
+
+// The pair lists of a rulebook built without them, on first use by the convs
+// that walk them (and the pair and statistics downloads).
 trellis_status rulebook_ensure_lists(Backend * be, const trellis_sparse_rulebook * rc) {
     auto * r = const_cast<trellis_sparse_rulebook *>(rc);
     if (r->pair_dst.ptr != nullptr) return TRELLIS_STATUS_OK;
-    DevMem counts, off, src, dst;
-    trellis_status st = dev_alloc(be, (size_t) r->n_tiles * 27 * 4, &counts);
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) r->n_tiles * 27 * 4, &off);
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) r->n_tiles * kMapTile * 27 * 4, &src);
-    if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) r->n_tiles * kMapTile * 27, &dst);
-    if (st == TRELLIS_STATUS_OK) {
-        stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
-        st = hip_status(be,
-                        launch_map_lists((const int32_t *) r->rows.ptr, r->n, (int32_t *) counts.ptr,
-                                         (int32_t *) off.ptr, (int32_t *) src.ptr, (uint8_t *) dst.ptr,
-                                         (int32_t *) r->counters.ptr, be->stream),
-                        "pair lists");
-        stage_end(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
-    }
+    PairLists lists;
+    trellis_status st = alloc_lists(be, r, &lists);
+    if (st != TRELLIS_STATUS_OK) return st;
+    stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
+    st = hip_status(be,
+                    launch_map_lists((const int32_t *) r->rows.ptr, r->n, lists, (int32_t *) r->counters.ptr,
+                                     be->stream),
+                    "pair lists");
+    stage_end(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
     if (st != TRELLIS_STATUS_OK) {
-        for (DevMem * m : {&counts, &off, &src, &dst}) dev_release(be, m);
-        return st;
+        for (DevMem * m : {&r->tile_counts, &r->tile_off, &r->pair_src, &r->pair_dst}) dev_release(be, m);
     }
-    r->tile_counts = counts;
-    r->tile_off = off;
-    r->pair_src = src;
-    r->pair_dst = dst;
-    return TRELLIS_STATUS_OK;
+    return st;
+}
+
+// The row table of a rulebook built as pair lists, on first use by what reads it.
+trellis_status rulebook_ensure_rows(Backend * be, const trellis_sparse_rulebook * rc) {
+    auto * r = const_cast<trellis_sparse_rulebook *>(rc);
+    if (r->rows.ptr != nullptr) return TRELLIS_STATUS_OK;
+    trellis_status st = dev_alloc(be, (size_t) r->n * kMapRow * 4, &r->rows);
+    if (st != TRELLIS_STATUS_OK) return st;
+    stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
+    st = hip_status(be,
+                    launch_list_rows((const uint32_t *) r->mask.ptr, r->n, (const int32_t *) r->tile_off.ptr,
+                                     (const int32_t *) r->pair_src.ptr, (int32_t *) r->rows.ptr, be->stream),
+                    "neighbour rows");
+    stage_end(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
+    if (st != TRELLIS_STATUS_OK) dev_release(be, &r->rows);
+    return st;
 }
 
 // The mask order costs 15 us (four launches) and 18 us more per million rows,
@@ -972,8 +995,9 @@ int64_t next_pow2(int64_t v) {
     return p;
 }
 
-// Builds the brick hash and the kernel map (neighbour rows and masks) for
-// device coordinates `coords` on the backend stream.
+// Builds the brick hash and the kernel map (masks, and neighbour rows, or pair
+// lists under the 16-bit COMPACT policy, whose convs walk them) for device
+// coordinates `coords` on the backend stream.
 trellis_status rulebook_build_device(Backend * be, const int32_t * coords, int64_t n, trellis_sparse_rulebook * r) {
     hipStream_t s = be->stream;
     r->n = n;
@@ -981,6 +1005,8 @@ trellis_status rulebook_build_device(Backend * be, const int32_t * coords, int64
     r->table_slots = std::max<int64_t>(64, next_pow2(2 * n));
     r->n_tiles = (n + kMapTile - 1) / kMapTile;
     const size_t slots = (size_t) r->table_slots;
+    const bool compact =
+        be->policy.conv_algo == TRELLIS_SPARSE_HIP_CONV_COMPACT && be->policy.compute_dtype != kF32;
     struct Need {
         DevMem * m;
         size_t bytes;
@@ -988,11 +1014,16 @@ trellis_status rulebook_build_device(Backend * be, const int32_t * coords, int64
         {&r->table, slots * 16},
         {&r->pool, (size_t) (pool_empty_brick(n) + 1) * kBrickCells * 4},
         {&r->counters, kCounterInts * 4},
-        {&r->rows, (size_t) n * kMapRow * 4},
+        {&r->rows, compact ? 0 : (size_t) n * kMapRow * 4},
         {&r->mask, (size_t) n * 4},
     };
     for (const Need & q : need) {
         const trellis_status st = dev_alloc(be, q.bytes, q.m);
+        if (st != TRELLIS_STATUS_OK) return st;
+    }
+    PairLists lists;
+    if (compact) {
+        const trellis_status st = alloc_lists(be, r, &lists);
         if (st != TRELLIS_STATUS_OK) return st;
     }
     stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_HASH);
@@ -1004,9 +1035,8 @@ trellis_status rulebook_build_device(Backend * be, const int32_t * coords, int64
                                     r->table_slots, (int32_t *) r->pool.ptr, (int32_t *) r->counters.ptr, s));
     stage_end(be, TRELLIS_SPARSE_HIP_STAGE_HASH);
     stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
-    TSH_TRY(be, launch_map_rows(coords, n, (const uint64_t *) r->table.ptr, r->table_slots,
-                                (const int32_t *) r->pool.ptr, (int32_t *) r->rows.ptr, (uint32_t *) r->mask.ptr,
-                                (int32_t *) r->counters.ptr, s));
+    TSH_TRY(be, launch_map(coords, n, (const uint64_t *) r->table.ptr, r->table_slots, (const int32_t *) r->pool.ptr,
+                           (int32_t *) r->rows.ptr, (uint32_t *) r->mask.ptr, lists, (int32_t *) r->counters.ptr, s));
     stage_end(be, TRELLIS_SPARSE_HIP_STAGE_MAP);
     if (be->policy.reject_duplicates) {
         int32_t flags[4] = {0, 0, 0, 0};
@@ -1080,8 +1110,12 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
     // an offset by zeros, so weights that are not finite, whose products would
     // be NaN where the reference skips the offset, run one that multiplies
     // valid pairs only: the compacted one, or the VALU one (with fp32 weights).
-    if (algo == TRELLIS_SPARSE_HIP_CONV_AUTO) {
-        // The sorted schedule takes every MFMA shape with Ci % 64 == 0.
+    if (algo == TRELLIS_SPARSE_HIP_CONV_AUTO ||
+        (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT && ci == 64 && co == 64)) {
+        // The sorted schedule takes every MFMA shape with Ci % 64 == 0; and 64 ->
+        // 64 under the COMPACT policy too, where a unit of 128 pairs has two K
+        // steps and adding its sums to the tile's in LDS costs more than its
+        // MFMAs (5,000 rows: 10 us, compacted 49; 419,340: 120 and 291).
         algo = TRELLIS_SPARSE_HIP_CONV_COMPACT;
         if (conv_sorted_supported(dt, ci, co, n)) {
             st = get_weight(be, weight, wcount, kLayoutConvMfmaGrouped, ci, co, &w, &finite);
@@ -1117,6 +1151,16 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
     }
     hipError_t err;
     if (algo == TRELLIS_SPARSE_HIP_CONV_MASKED || algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
+        // (Without memory for the rows a map of pair lists is walked as it is.)
+        if (sorted) {
+            st = rulebook_ensure_rows(be, rulebook);
+            if (st == TRELLIS_STATUS_OUT_OF_MEMORY) {
+                be->last_error.clear();
+                st = TRELLIS_STATUS_OK;
+                sorted = false;
+            }
+            if (st != TRELLIS_STATUS_OK) return st;
+        }
         if (sorted) {
             // Where the order's memory does not fit, the rows are taken in their
             // own: the same sums, more of the multiplied rows absent.
@@ -1127,6 +1171,8 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
             }
         } else if (algo == TRELLIS_SPARSE_HIP_CONV_COMPACT) {
             st = rulebook_ensure_lists(be, rulebook);
+        } else {
+            st = rulebook_ensure_rows(be, rulebook);
         }
         if (st != TRELLIS_STATUS_OK) return st;
         stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_CONV);
@@ -1150,6 +1196,7 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
         stage_end(be, TRELLIS_SPARSE_HIP_STAGE_CONV);
     } else {
         st = get_weight(be, weight, wcount, kLayoutConvF32, ci, co, &w);
+        if (st == TRELLIS_STATUS_OK) st = rulebook_ensure_rows(be, rulebook);
         if (st != TRELLIS_STATUS_OK) return st;
         stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_CONV);
         err = launch_conv_generic(dt, feats->ptr, (const int32_t *) rulebook->rows.ptr, (const float *) w,
@@ -1810,6 +1857,7 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
         st = hip_status(be, err, "flex_dual_grid_mesh vertices");
     }
     if (st == TRELLIS_STATUS_OK) st = rulebook_build_device(be, coords, n, r);
+    if (st == TRELLIS_STATUS_OK) st = rulebook_ensure_rows(be, r);
     if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 4, &counts);
     if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, (size_t) n * 4, &first);
     if (st == TRELLIS_STATUS_OK) st = dev_alloc(be, 16, &total);
@@ -2142,7 +2190,8 @@ trellis_status trellis_sparse_hip_download_neighbors(trellis_sparse_backend * ba
     Backend * be = tsh::as_backend(backend);
     tsh::select_device(be);
     tsh::DevMem nbr;
-    const trellis_status st = tsh::dev_alloc(be, (size_t) n * 27 * 4, &nbr);
+    trellis_status st = tsh::rulebook_ensure_rows(be, rulebook);
+    if (st == TRELLIS_STATUS_OK) st = tsh::dev_alloc(be, (size_t) n * 27 * 4, &nbr);
     if (st != TRELLIS_STATUS_OK) return st;
     hipError_t err = tsh::launch_rows_nbr((const int32_t *) rulebook->rows.ptr, n, (int32_t *) nbr.ptr, be->stream);
     if (err == hipSuccess)

@@ -212,18 +212,127 @@ __global__ void __launch_bounds__(kBlock) k_voxel_insert(const int4 * __restrict
     atomicMax(&pool[(int64_t) b * kBrickCells + cell], (int32_t) i);
 }
 
+// Per-tile pair lists of a 256-row tile whose block's lanes hold a row's
+// neighbours (nb) and mask (m, 0 past the last row) each:
+//  1. per-offset pair counts of the tile (wavefront ballots);
+//  2. the per-(tile, offset) counts and list starts, and the pair lists,
+//     destination ascending within each (tile, offset).
+// Tile t owns the fixed region [t * 256 * 27, (t + 1) * 256 * 27) of the
+// pair arrays (the most pairs 256 rows can have), so no tile waits for the
+// counts of the tiles before it; the lists of a tile are packed from the
+// region's start, the centre offset (k = 13) first, then the others in
+// order.  Every row has exactly one centre neighbour (itself, or the last
+// duplicate of its coordinates), so the centre list holds the tile's rows in
+// order, starting at the region's start: a consumer can find it without the
+// tile's counts.
+template <int N>
+__device__ __forceinline__ void write_lists(uint32_t m, const int32_t (&nb)[N], const PairLists & lists,
+                                            int32_t * counters) {
+    __shared__ int32_t s_wave_cnt[27][kBlock / 64];
+    __shared__ int32_t s_koff[27];
+    const int t = threadIdx.x;
+    const int lane = lane_id();
+    const int wave = t >> 6;
+    const int64_t tile = blockIdx.x;
+    // Rows of this wavefront with a neighbour at k (the ranks are recomputed
+    // from the same ballots when the pairs are written).
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+        const uint64_t bal = __ballot((m >> k) & 1u);
+        if (lane == 0) s_wave_cnt[k][wave] = __popcll(bal);
+    }
+    __syncthreads();
+    if (t < 64) {
+        // Tile counts per offset and their exclusive scan in packing order:
+        // lane 0 takes the centre offset, lanes 1..26 the others in order.
+        const int k = t == 0 ? 13 : (t <= 13 ? t - 1 : t);
+        int32_t cnt = 0;
+        if (t < 27) {
+#pragma unroll
+            for (int w = 0; w < kBlock / 64; ++w) cnt += s_wave_cnt[k][w];
+            lists.tile_counts[tile * 27 + k] = cnt;
+        }
+        int32_t incl = cnt;
+#pragma unroll
+        for (int d = 1; d < 32; d <<= 1) {
+            const int32_t o = __shfl_up(incl, d);
+            if (lane >= d) incl += o;
+        }
+        if (t < 27) s_koff[k] = incl - cnt;
+        // Layout statistics for the convs with 256-column blocks: this
+        // tile's offsets with pairs, and with more than half the tile.
+        const int with = __popcll(__ballot(cnt > 0));
+        const int busy = __popcll(__ballot(cnt > kBlock / 2));
+        if (t == 0) {
+            const int slot = (int) (blockIdx.x % kLayoutSlots);
+            atomicAdd(&counters[kLayoutStats + slot], with);
+            atomicAdd(&counters[kLayoutStats + kLayoutSlots + slot], busy);
+        }
+    }
+    __syncthreads();
+    const int64_t base = tile * kBlock * 27;
+    if (t < 27) lists.tile_off[tile * 27 + t] = (int32_t) (base + s_koff[t]);
+    // Every lane takes part in the ballots; rows past n have no neighbours.
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+        const uint64_t bal = __ballot((m >> k) & 1u);
+        if ((m >> k) & 1u) {
+            int64_t pos = base + s_koff[k] + __popcll(bal & lt);
+            for (int w = 0; w < wave; ++w) pos += s_wave_cnt[k][w];
+            lists.pair_src[pos] = nb[k];
+            lists.pair_dst[pos] = (uint8_t) t;
+        }
+    }
+}
+
+// A block's 256 rows of the row table, a lane holding one each.
+__device__ __forceinline__ void write_rows(uint32_t m, const int32_t (&nb)[27], int32_t * rows, int64_t n) {
+    // The rows leave through LDS, 16 of the wavefront's at a time (1.8 KB per
+    // wavefront, so that the LDS does not bound the occupancy), as
+    // consecutive 16-byte pieces; a lane writing its own row's pieces 112
+    // bytes apart took 0.276 instead of 0.229 ms on 3,788,747 rows.
+    __shared__ int4 s_rows[kBlock / 64][16 * (kMapRow / 4)];
+    const int lane = lane_id(), wave = threadIdx.x >> 6;
+    const int64_t wave0 = (int64_t) blockIdx.x * kBlock + wave * 64;
+    int4 * const stage = s_rows[wave];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        if ((lane >> 4) == g) {
+            int4 * at = stage + (lane & 15) * (kMapRow / 4);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) at[c] = int4{nb[4 * c], nb[4 * c + 1], nb[4 * c + 2], nb[4 * c + 3]};
+            at[6] = int4{nb[24], nb[25], nb[26], (int32_t) m};
+        }
+        // One wavefront's LDS operations run in order; the fence only keeps
+        // the compiler from moving them.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int64_t row0 = wave0 + g * 16;
+        const int64_t left = (n - row0) * (kMapRow / 4);
+        int4 * out = (int4 *) (rows + row0 * kMapRow);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int e = j * 64 + lane;
+            if (e < 16 * (kMapRow / 4) && e < left) out[e] = stage[e];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+}
+
 // Kernel map: one lane finds its voxel's 27 neighbour rows (a few brick probes
 // plus 9 z-row pool reads), keeps them in registers and writes them with the
-// row mask as seven 16-byte pieces.  (Until the convs read this table, the
-// kernel packed per-tile pair lists instead, which took 27 ballots, ranks and
-// scattered stores per wavefront.)
+// row mask as seven 16-byte pieces, or (LISTS) the tile's pair lists, whose 27
+// ballots, ranks and scattered stores per wavefront only the convs that walk
+// them need.  Either can be made from the other later.  With its hash, 419,340
+// rows: rows 49 us, lists 57, both in one launch 82; 3,788,747: 402, 362, 703.
 // Seven wavefronts per SIMD (at most 72 registers): 4 % faster than six on
 // config 3's map, while eight spill.
-__global__ void __launch_bounds__(kBlock, 7) k_map_rows(const int4 * __restrict__ coords, int64_t n,
-                                                        const uint64_t * __restrict__ table, uint64_t hmask,
-                                                        const int32_t * __restrict__ pool, int32_t empty_brick,
-                                                        int32_t * __restrict__ rows, uint32_t * __restrict__ mask_out,
-                                                        int32_t * __restrict__ counters) {
+template <bool LISTS>
+__global__ void __launch_bounds__(kBlock, 7) k_map(const int4 * __restrict__ coords, int64_t n,
+                                                   const uint64_t * __restrict__ table, uint64_t hmask,
+                                                   const int32_t * __restrict__ pool, int32_t empty_brick,
+                                                   int32_t * __restrict__ rows, uint32_t * __restrict__ mask_out,
+                                                   PairLists lists, int32_t * __restrict__ counters) {
     const int64_t i = (int64_t) blockIdx.x * kBlock + threadIdx.x;
     uint32_t m = 0;
     int32_t nb[27];
@@ -317,61 +426,17 @@ __global__ void __launch_bounds__(kBlock, 7) k_map_rows(const int4 * __restrict_
         // other value means duplicate coordinates.
         if (nb[13] != (int32_t) i) atomicOr(&counters[1], 1);
     }
-    // The rows leave through LDS, 16 of the wavefront's at a time (1.8 KB per
-    // wavefront, so that the LDS does not bound the occupancy), as
-    // consecutive 16-byte pieces; a lane writing its own row's pieces 112
-    // bytes apart took 0.276 instead of 0.229 ms on 3,788,747 rows.
-    __shared__ int4 s_rows[kBlock / 64][16 * (kMapRow / 4)];
-    const int lane = lane_id(), wave = threadIdx.x >> 6;
-    const int64_t wave0 = (int64_t) blockIdx.x * kBlock + wave * 64;
-    int4 * const stage = s_rows[wave];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        if ((lane >> 4) == g) {
-            int4 * at = stage + (lane & 15) * (kMapRow / 4);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) at[c] = int4{nb[4 * c], nb[4 * c + 1], nb[4 * c + 2], nb[4 * c + 3]};
-            at[6] = int4{nb[24], nb[25], nb[26], (int32_t) m};
-        }
-        // One wavefront's LDS operations run in order; the fence only keeps
-        // the compiler from moving them.
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        const int64_t row0 = wave0 + g * 16;
-        const int64_t left = (n - row0) * (kMapRow / 4);
-        int4 * out = (int4 *) (rows + row0 * kMapRow);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int e = j * 64 + lane;
-            if (e < 16 * (kMapRow / 4) && e < left) out[e] = stage[e];
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if constexpr (LISTS) {
+        write_lists(m, nb, lists, counters);
+    } else {
+        write_rows(m, nb, rows, n);
     }
 }
 
-// Per-tile pair lists from the row table; one block = one 256-row tile:
-//  1. per-offset pair counts of the tile (wavefront ballots);
-//  2. the per-(tile, offset) counts and list starts, and the pair lists,
-//     destination ascending within each (tile, offset).
-// Tile t owns the fixed region [t * 256 * 27, (t + 1) * 256 * 27) of the
-// pair arrays (the most pairs 256 rows can have), so no tile waits for the
-// counts of the tiles before it; the lists of a tile are packed from the
-// region's start, the centre offset (k = 13) first, then the others in
-// order.  Every row has exactly one centre neighbour (itself, or the last
-// duplicate of its coordinates), so the centre list holds the tile's rows in
-// order, starting at the region's start: a consumer can find it without the
-// tile's counts.
-__global__ void __launch_bounds__(kBlock) k_map_lists(const int32_t * __restrict__ rows, int64_t n,
-                                                      int32_t * __restrict__ tile_counts,
-                                                      int32_t * __restrict__ tile_off,
-                                                      int32_t * __restrict__ pair_src,
-                                                      uint8_t * __restrict__ pair_dst, int32_t * __restrict__ counters) {
-    __shared__ int32_t s_wave_cnt[27][kBlock / 64];
-    __shared__ int32_t s_koff[27];
-    const int t = threadIdx.x;
-    const int lane = lane_id();
-    const int wave = t >> 6;
-    const int64_t tile = blockIdx.x;
-    const int64_t i = tile * kBlock + t;
+// The pair lists from the row table.
+__global__ void __launch_bounds__(kBlock) k_map_lists(const int32_t * __restrict__ rows, int64_t n, PairLists lists,
+                                                      int32_t * __restrict__ counters) {
+    const int64_t i = (int64_t) blockIdx.x * kBlock + threadIdx.x;
     uint32_t m = 0;
     int32_t nb[28];
     if (i < n) {
@@ -386,56 +451,35 @@ __global__ void __launch_bounds__(kBlock) k_map_lists(const int32_t * __restrict
         }
         m = (uint32_t) nb[27];
     }
-    // Rows of this wavefront with a neighbour at k (the ranks are recomputed
-    // from the same ballots when the pairs are written).
+    write_lists(m, nb, lists, counters);
+}
+
+// The row table from the pair lists: a row's rank in its tile's list of an
+// offset is the number of earlier rows with a neighbour there.
+__global__ void __launch_bounds__(kBlock) k_list_rows(const uint32_t * __restrict__ mask, int64_t n,
+                                                      const int32_t * __restrict__ tile_off,
+                                                      const int32_t * __restrict__ pair_src,
+                                                      int32_t * __restrict__ rows) {
+    __shared__ int32_t s_cnt[27][kBlock / 64];
+    const int lane = lane_id(), wave = threadIdx.x >> 6;
+    const int64_t tile = blockIdx.x, i = tile * kBlock + threadIdx.x;
+    const uint32_t m = i < n ? mask[i] : 0u;
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 #pragma unroll
     for (int k = 0; k < 27; ++k) {
         const uint64_t bal = __ballot((m >> k) & 1u);
-        if (lane == 0) s_wave_cnt[k][wave] = __popcll(bal);
+        if (lane == 0) s_cnt[k][wave] = __popcll(bal);
     }
     __syncthreads();
-    if (t < 64) {
-        // Tile counts per offset and their exclusive scan in packing order:
-        // lane 0 takes the centre offset, lanes 1..26 the others in order.
-        const int k = t == 0 ? 13 : (t <= 13 ? t - 1 : t);
-        int32_t cnt = 0;
-        if (t < 27) {
-#pragma unroll
-            for (int w = 0; w < kBlock / 64; ++w) cnt += s_wave_cnt[k][w];
-            tile_counts[tile * 27 + k] = cnt;
-        }
-        int32_t incl = cnt;
-#pragma unroll
-        for (int d = 1; d < 32; d <<= 1) {
-            const int32_t o = __shfl_up(incl, d);
-            if (lane >= d) incl += o;
-        }
-        if (t < 27) s_koff[k] = incl - cnt;
-        // Layout statistics for the convs with 256-column blocks: this
-        // tile's offsets with pairs, and with more than half the tile.
-        const int with = __popcll(__ballot(cnt > 0));
-        const int busy = __popcll(__ballot(cnt > kBlock / 2));
-        if (t == 0) {
-            const int slot = (int) (blockIdx.x % kLayoutSlots);
-            atomicAdd(&counters[kLayoutStats + slot], with);
-            atomicAdd(&counters[kLayoutStats + kLayoutSlots + slot], busy);
-        }
-    }
-    __syncthreads();
-    const int64_t base = tile * kBlock * 27;
-    if (t < 27) tile_off[tile * 27 + t] = (int32_t) (base + s_koff[t]);
-    // Every lane takes part in the ballots; rows past n have no neighbours.
+    int32_t nb[27];
 #pragma unroll
     for (int k = 0; k < 27; ++k) {
         const uint64_t bal = __ballot((m >> k) & 1u);
-        if ((m >> k) & 1u) {
-            int64_t pos = base + s_koff[k] + __popcll(bal & lt);
-            for (int w = 0; w < wave; ++w) pos += s_wave_cnt[k][w];
-            pair_src[pos] = nb[k];
-            pair_dst[pos] = (uint8_t) t;
-        }
+        int32_t at = tile_off[tile * 27 + k] + __popcll(bal & lt);
+        for (int w = 0; w < wave; ++w) at += s_cnt[k][w];
+        nb[k] = ((m >> k) & 1u) ? pair_src[at] : -1;
     }
+    write_rows(m, nb, rows, n);
 }
 
 int grid_for(int64_t count, int block, int cap = 65536) {
@@ -481,18 +525,31 @@ hipError_t launch_voxel_insert(const int32_t * coords, int64_t n, const uint64_t
     return hipGetLastError();
 }
 
-hipError_t launch_map_rows(const int32_t * coords, int64_t n, const uint64_t * table, int64_t slots,
-                           const int32_t * pool, int32_t * rows, uint32_t * mask, int32_t * counters, hipStream_t s) {
-    const int64_t blocks = (n + kBlock - 1) / kBlock;
-    k_map_rows<<<(unsigned) blocks, kBlock, 0, s>>>((const int4 *) coords, n, table, (uint64_t) (slots - 1), pool,
-                                                    (int32_t) pool_empty_brick(n), rows, mask, counters);
+hipError_t launch_map(const int32_t * coords, int64_t n, const uint64_t * table, int64_t slots, const int32_t * pool,
+                      int32_t * rows, uint32_t * mask, const PairLists & lists, int32_t * counters, hipStream_t s) {
+    const unsigned blocks = (unsigned) ((n + kBlock - 1) / kBlock);
+    const int32_t empty = (int32_t) pool_empty_brick(n);
+    if (rows == nullptr) {
+        k_map<true><<<blocks, kBlock, 0, s>>>((const int4 *) coords, n, table, (uint64_t) (slots - 1), pool, empty, rows,
+                                              mask, lists, counters);
+    } else {
+        k_map<false><<<blocks, kBlock, 0, s>>>((const int4 *) coords, n, table, (uint64_t) (slots - 1), pool, empty,
+                                               rows, mask, lists, counters);
+    }
     return hipGetLastError();
 }
 
-hipError_t launch_map_lists(const int32_t * rows, int64_t n, int32_t * tile_counts, int32_t * tile_off,
-                            int32_t * pair_src, uint8_t * pair_dst, int32_t * counters, hipStream_t s) {
+hipError_t launch_map_lists(const int32_t * rows, int64_t n, const PairLists & lists, int32_t * counters,
+                            hipStream_t s) {
     const int64_t blocks = (n + kBlock - 1) / kBlock;
-    k_map_lists<<<(unsigned) blocks, kBlock, 0, s>>>(rows, n, tile_counts, tile_off, pair_src, pair_dst, counters);
+    k_map_lists<<<(unsigned) blocks, kBlock, 0, s>>>(rows, n, lists, counters);
+    return hipGetLastError();
+}
+
+hipError_t launch_list_rows(const uint32_t * mask, int64_t n, const int32_t * tile_off, const int32_t * pair_src,
+                            int32_t * rows, hipStream_t s) {
+    const int64_t blocks = (n + kBlock - 1) / kBlock;
+    k_list_rows<<<(unsigned) blocks, kBlock, 0, s>>>(mask, n, tile_off, pair_src, rows);
     return hipGetLastError();
 }
 

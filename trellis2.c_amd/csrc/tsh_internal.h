@@ -151,7 +151,8 @@ struct trellis_sparse_rulebook {
     tsh::DevMem rows;        // int32  [n][kMapRow]: 27 neighbour rows (-1 = none), then the mask
     tsh::DevMem mask;        // uint32 [n] bit k set when rows[i][k] >= 0
     int64_t n_tiles;         // ceil(n / kMapTile)
-    // Pair lists (built for the kernels that walk them).
+    // Pair lists.  Under the 16-bit COMPACT policy the map is built as these and
+    // the rows follow from them on first use, otherwise the other way round.
     tsh::DevMem tile_counts; // int32  [n_tiles][27]
     tsh::DevMem tile_off;    // int32  [n_tiles][27] start of (tile, k) in the pair arrays
     tsh::DevMem pair_src;    // int32  [n_tiles][kMapTile * 27]: per tile, offsets ascending, dst ascending
@@ -193,14 +194,24 @@ int64_t pool_empty_brick(int64_t n);
 
 hipError_t launch_voxel_insert(const int32_t * coords, int64_t n, const uint64_t * table,
                                int64_t slots, int32_t * pool, int32_t * counters, hipStream_t s);
-// Neighbour rows and masks of every voxel.
-hipError_t launch_map_rows(const int32_t * coords, int64_t n, const uint64_t * table, int64_t slots,
-                           const int32_t * pool, int32_t * rows, uint32_t * mask, int32_t * counters, hipStream_t s);
-// Per-(tile, offset) counts and list starts and the pair lists from the row
-// table.  Tile t's lists fill the start of its region
-// [t * kMapTile * 27, (t + 1) * kMapTile * 27) of the pair arrays.
-hipError_t launch_map_lists(const int32_t * rows, int64_t n, int32_t * tile_counts, int32_t * tile_off,
-                            int32_t * pair_src, uint8_t * pair_dst, int32_t * counters, hipStream_t s);
+// Per-(tile, offset) counts and list starts, and the pair lists.  Tile t's lists
+// fill the start of its region [t * kMapTile * 27, (t + 1) * kMapTile * 27) of
+// the pair arrays.
+struct PairLists {
+    int32_t * tile_counts = nullptr;
+    int32_t * tile_off = nullptr;
+    int32_t * pair_src = nullptr;
+    uint8_t * pair_dst = nullptr;
+};
+// Every voxel's mask and its neighbour rows, or with rows == nullptr the pair
+// lists.
+hipError_t launch_map(const int32_t * coords, int64_t n, const uint64_t * table, int64_t slots, const int32_t * pool,
+                      int32_t * rows, uint32_t * mask, const PairLists & lists, int32_t * counters, hipStream_t s);
+// The pair lists from the row table, and the row table from the pair lists.
+hipError_t launch_map_lists(const int32_t * rows, int64_t n, const PairLists & lists, int32_t * counters,
+                            hipStream_t s);
+hipError_t launch_list_rows(const uint32_t * mask, int64_t n, const int32_t * tile_off, const int32_t * pair_src,
+                            int32_t * rows, hipStream_t s);
 // The dense [n][27] neighbour table of the row table.
 hipError_t launch_rows_nbr(const int32_t * rows, int64_t n, int32_t * nbr, hipStream_t s);
 
