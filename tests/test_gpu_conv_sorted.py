@@ -80,6 +80,19 @@ def test_block_edges(backends, n, ci, co):
     assert err(y, sh.storage_round(orc.Rulebook(coords).conv(x, w, b, ci, co), dtype)) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("n", [1, 31, 63, 64, 65, 127, 128, 129, 1000])
+@pytest.mark.parametrize("ci,co", [(32, 16), (96, 32), (32, 64), (96, 128), (160, 192)])
+def test_masked_block_edges(backends, n, ci, co):
+    """The widths beside the sorted kernel's (odd multiples of 32), on the masked kernel."""
+    dtype = sh.BF16 if n % 2 else sh.F16
+    rng = np.random.default_rng(n * 7 + ci + co)
+    coords = shell(n)
+    x = sh.storage_round(rng.standard_normal((n, ci)), dtype)
+    w, b = weights(rng, ci, co, dtype), (0.1 * rng.standard_normal(co)).astype(np.float32)
+    y = run(backends[dtype], coords, x, w, b, ci, co)
+    assert err(y, sh.storage_round(orc.Rulebook(coords).conv(x, w, b, ci, co), dtype)) <= TOL[dtype]
+
+
 # Row counts that take each block shape at 256 and 128 channels (64 x 64 up to 256 x 256), sampled rows.
 @pytest.mark.parametrize("ci,co,n", [(64, 256, 3000), (64, 256, 9000), (64, 256, 14648), (64, 512, 14648),
                                      (64, 1024, 6000), (64, 1024, 8100), (64, 1024, 9000), (64, 1024, 12000),

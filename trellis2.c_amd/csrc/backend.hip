@@ -1189,9 +1189,8 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
                                           ci, co, be->stream, epi,
                                           (const int32_t *) rulebook->counters.ptr + kLayoutStats);
         } else {
-            err = launch_conv_mfma_masked(dt, feats->ptr, (const int32_t *) rulebook->rows.ptr,
-                                          (const uint32_t *) rulebook->mask.ptr, w, (const float *) bd, out->ptr, n,
-                                          ci, co, be->stream);
+            err = launch_conv_mfma_masked(dt, feats->ptr, (const int32_t *) rulebook->rows.ptr, w, (const float *) bd,
+                                          out->ptr, n, ci, co, be->stream);
         }
         stage_end(be, TRELLIS_SPARSE_HIP_STAGE_CONV);
     } else {
