@@ -28,7 +28,8 @@ def backends():
 
 @pytest.mark.parametrize("silu", [False, True])
 @pytest.mark.parametrize("n,ci,co", [(1, 64, 128), (63, 128, 256), (64, 192, 128), (129, 64, 384), (257, 320, 256),
-                                     (5003, 64, 256), (20000, 64, 512), (33000, 64, 256), (131080, 64, 128)])
+                                     (5003, 64, 256), (20000, 64, 512), (33000, 64, 256), (131080, 64, 128),
+                                     (5003, 512, 512), (41000, 64, 256), (131080, 64, 512), (524300, 64, 128)])
 def test_linear_vs_oracle(backends, n, ci, co, silu):
     dtype = sh.F16 if n % 2 else sh.BF16
     be = backends[dtype]

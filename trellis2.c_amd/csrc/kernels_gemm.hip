@@ -151,9 +151,26 @@ hipError_t launch_dt(const void * x, const void * w16, const float * bias, const
     // 4096 with SiLU on 18,216 0.17 (0.25), 256 -> 1024 with SiLU on 300,000
     // 0.36 (0.42), 128 -> 128 on 1,000,000 0.118 (0.134); 2048 -> 512 on 5,003
     // rows: 128 x 256 0.028, 128 x 128 0.021.
-    if (co % 256 == 0 && blocks(128, 256) >= cus) return TSH_GEMM(128, 256, 2, 2, 3);
-    if (co % 256 != 0 && blocks(256, 128) >= 2 * (int64_t) cus) return TSH_GEMM(256, 128, 4, 1, 3);
-    if (5 * blocks(128, 128) >= 3 * (int64_t) cus) return TSH_GEMM(128, 128, 4, 1, 3);
+    // SiLU's exponentials are VALU work at a block's end, which weighs on short K
+    // loops: up to Ci = 256 and eight large blocks per CU smaller ones overlap it
+    // better (us, 128 x 256 / 128 x 128 / 64 x 128; k_linear_mfma: 256 -> 1024 on
+    // 12,000 rows 16.7 / 14.9 / 15.0; 15.6; 256 -> 256 on 80,000 24.8 / 21.9 /
+    // 24.4; 23.8, on 300,000 83 / 88 / 115; 101; 256 x 128 on 128 -> 384, 80,000
+    // rows 27.0 / 23.2 / 25.6; 26.5; 256 -> 1024 on 5,000 11.1 / 9.3 / 8.4; 11.1;
+    // 128 -> 128 on 40,000 - / 8.1 / 7.3; 8.9; but 1024 -> 4096 on 12,000 99 /
+    // 129).
+    const bool short_silu = silu && ci <= 256;
+    const int64_t b128 = blocks(128, 128);
+    if (co % 256 == 0 && blocks(128, 256) >= (short_silu ? 8 : 1) * (int64_t) cus) return TSH_GEMM(128, 256, 2, 2, 3);
+    if (co % 256 != 0 && blocks(256, 128) >= (short_silu ? 8 : 2) * (int64_t) cus) return TSH_GEMM(256, 128, 4, 1, 3);
+    if (5 * b128 >= 3 * (int64_t) cus && !(short_silu && 2 * b128 < 3 * (int64_t) cus)) {
+        // One block on a CU has room for a fourth slot, which pays on deep rows
+        // (2048 -> 512 on 5,000: 20.2 -> 18.4 us, with SiLU 21.4 -> 19.4; 1024 ->
+        // 256 on 12,000 11.7 -> 11.4; with more blocks 4096 -> 1024 on 5,000 52
+        // -> 56).
+        if (ci >= 512 && b128 <= cus) return TSH_GEMM(128, 128, 4, 1, 4);
+        return TSH_GEMM(128, 128, 4, 1, 3);
+    }
     return TSH_GEMM(64, 128, 4, 1, 4);
 #undef TSH_GEMM
 }
