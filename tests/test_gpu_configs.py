@@ -9,7 +9,10 @@ tests/test_sparse_decoder_backend.c:16-24 (|a-b| <= 2e-2 max(1,|a|,|b|)).
 For configs 4 and 5 the stride is 255 rows plus the last row, so every
 256-row map tile (the kernels' unit of work) holds at least one sampled row,
 including the last, partial tile, and the sampled positions within a tile
-cycle through all 256 (both half tiles of the 256-channel blocks).
+cycle through all 256 (both half tiles of the compacted kernel's 256-channel
+blocks).  The configurations run the AUTO policy (the sorted kernel); the
+deep-channel, layout and level tests also the COMPACT one, whose kernels they
+were shaped for.
 
   config 2  conv(128->128) -> LayerNorm -> SiLU -> conv(128->128) + skip, fp16,
             419,340 voxels: each fused launch against the oracle, the second
@@ -62,6 +65,16 @@ def backends():
     yield bes
     for b in bes.values():
         b.destroy()
+
+
+@pytest.fixture(scope="module")
+def schedules():
+    """Per storage type the backends of the AUTO policy (the sorted kernel) and the COMPACT one."""
+    bes = {dt: [sh.Backend(0, dt), sh.Backend(0, dt, conv_algo=sh.CONV_COMPACT)] for dt in (sh.F16, sh.BF16)}
+    yield bes
+    for pair in bes.values():
+        for b in pair:
+            b.destroy()
 
 
 def sample_rows(n, want):
@@ -150,44 +163,44 @@ DEEP_CASES = [(512, 128, 3001), (384, 128, 2000), (1024, 128, 1200), (512, 64, 2
 
 @pytest.mark.parametrize("dtype", [sh.BF16, sh.F16])
 @pytest.mark.parametrize("ci,co,n", DEEP_CASES)
-def test_conv_deep_channels_vs_oracle(backends, dtype, ci, co, n):
-    be = backends[dtype]
+def test_conv_deep_channels_vs_oracle(schedules, dtype, ci, co, n):
     coords = np.ascontiguousarray(wl.make_coords(1)[:n])
     rng = np.random.default_rng(ci + 3 * co + n + dtype)
     x = sh.storage_round(rng.standard_normal((n, ci)), dtype)
     w = sh.storage_round(rng.standard_normal((co, 27, ci)) / math.sqrt(27 * ci), dtype)
     bias = (0.1 * rng.standard_normal(co)).astype(np.float32)
     say(f"deep conv dtype={dtype} ci={ci} co={co} n={n}")
-    rb = be.build_rulebook(coords)
-    xb, yb = be.upload(x), be.alloc(n * co)
-    be.conv(rb, xb, w, bias, yb, ci, co)
-    got = be.download(yb).reshape(n, co)
     rows = sample_rows(n, 400 if ci * co <= 512 * 1024 else 120)
     exp = orc.Rulebook(coords).conv(x, w, bias, ci, co, rows=rows)
-    err = max_rel_err(got[rows[0]:rows[1]:rows[2]], exp)
-    say(f"deep conv dtype={dtype} ci={ci} co={co} n={n} rows={exp.shape[0]} max_rel_err={err:.3e}")
-    assert err <= TOL[dtype]
-    # Fused epilogues on the multi-block path (128-channel blocks only).
-    if co % 128 == 0:
-        res = sh.storage_round(rng.standard_normal((n, co)), dtype)
-        rs = be.upload(res)
-        be.conv_add(rb, xb, w, bias, rs, yb, ci, co)
-        got_add = be.download(yb).reshape(n, co)
-        e_add = sh.storage_round(orc.add(sh.storage_round(exp, dtype), res[rows[0]:rows[1]:rows[2]]), dtype)
-        err_add = max_rel_err(got_add[rows[0]:rows[1]:rows[2]], e_add)
-        say(f"deep conv_add dtype={dtype} ci={ci} co={co} max_rel_err={err_add:.3e}")
-        assert err_add <= TOL[dtype]
-    if co == 128:
-        gamma = (1 + 0.1 * rng.standard_normal(co)).astype(np.float32)
-        beta = (0.1 * rng.standard_normal(co)).astype(np.float32)
-        be.conv_norm(rb, xb, w, bias, gamma, beta, 1e-6, yb, ci, co, silu=True)
-        got_n = be.download(yb).reshape(n, co)
-        e_n = sh.storage_round(orc.row_norm(sh.storage_round(exp, dtype), gamma, beta, exp.shape[0], co, 1e-6,
-                                            silu=True), dtype)
-        err_n = max_rel_err(got_n[rows[0]:rows[1]:rows[2]], e_n)
-        say(f"deep conv_norm dtype={dtype} ci={ci} max_rel_err={err_n:.3e}")
-        assert err_n <= TOL[dtype]
-    rb.free()
+    res = sh.storage_round(rng.standard_normal((n, co)), dtype)
+    gamma = (1 + 0.1 * rng.standard_normal(co)).astype(np.float32)
+    beta = (0.1 * rng.standard_normal(co)).astype(np.float32)
+    for be in schedules[dtype]:
+        rb = be.build_rulebook(coords)
+        xb, yb = be.upload(x), be.alloc(n * co)
+        be.conv(rb, xb, w, bias, yb, ci, co)
+        got = be.download(yb).reshape(n, co)
+        err = max_rel_err(got[rows[0]:rows[1]:rows[2]], exp)
+        say(f"deep conv dtype={dtype} ci={ci} co={co} n={n} rows={exp.shape[0]} max_rel_err={err:.3e}")
+        assert err <= TOL[dtype]
+        # Fused epilogues on the multi-block path (128-channel blocks only).
+        if co % 128 == 0:
+            rs = be.upload(res)
+            be.conv_add(rb, xb, w, bias, rs, yb, ci, co)
+            got_add = be.download(yb).reshape(n, co)
+            e_add = sh.storage_round(orc.add(sh.storage_round(exp, dtype), res[rows[0]:rows[1]:rows[2]]), dtype)
+            err_add = max_rel_err(got_add[rows[0]:rows[1]:rows[2]], e_add)
+            say(f"deep conv_add dtype={dtype} ci={ci} co={co} max_rel_err={err_add:.3e}")
+            assert err_add <= TOL[dtype]
+        if co == 128:
+            be.conv_norm(rb, xb, w, bias, gamma, beta, 1e-6, yb, ci, co, silu=True)
+            got_n = be.download(yb).reshape(n, co)
+            e_n = sh.storage_round(orc.row_norm(sh.storage_round(exp, dtype), gamma, beta, exp.shape[0], co, 1e-6,
+                                                silu=True), dtype)
+            err_n = max_rel_err(got_n[rows[0]:rows[1]:rows[2]], e_n)
+            say(f"deep conv_norm dtype={dtype} ci={ci} max_rel_err={err_n:.3e}")
+            assert err_n <= TOL[dtype]
+        rb.free()
 
 
 def mixed_density_sets(rng):
@@ -205,16 +218,16 @@ def mixed_density_sets(rng):
 
 @pytest.mark.parametrize("dtype", [sh.BF16, sh.F16])
 @pytest.mark.parametrize("ci,co", [(128, 256), (256, 512), (512, 256), (256, 1024), (512, 2048)])
-def test_conv_layouts_bitexact(backends, dtype, ci, co):
-    """Co % 256 == 0 runs the 256-column layout on dense sets and the
-    128-column one on sparse sets (the kernel map's statistics decide).  The
+def test_conv_layouts_bitexact(schedules, dtype, ci, co):
+    """Under the COMPACT policy Co % 256 == 0 runs the 256-column layout on
+    dense sets and the 128-column one on sparse sets (the kernel map's
+    statistics decide); under AUTO the set's size chooses the block shape.  The
     box alone takes the first, the union of box and sparse part the second:
     the union's rows must equal, bit for bit, the same rows computed from
     each part alone (a row's sums are formed in the same order in both
     layouts, and the parts are too far apart to be neighbours), with and
     without the residual epilogue (in place), and match the oracle on a
     sample."""
-    be = backends[dtype]
     rng = np.random.default_rng(ci + co)
     box, sparse = mixed_density_sets(rng)
     both = np.ascontiguousarray(np.concatenate([box, sparse]))
@@ -225,7 +238,7 @@ def test_conv_layouts_bitexact(backends, dtype, ci, co):
     res = sh.storage_round(rng.standard_normal((n, co)), dtype)
     say(f"conv layouts dtype={dtype} ci={ci} co={co} box={nb} sparse={n - nb}")
 
-    def run(coords, xs, rs):
+    def run(be, coords, xs, rs):
         rb = be.build_rulebook(coords)
         m = coords.shape[0]
         xb, yb = be.upload(xs), be.alloc(m * co)
@@ -237,28 +250,28 @@ def test_conv_layouts_bitexact(backends, dtype, ci, co):
         rb.free()
         return plain, added
 
-    p_all, a_all = run(both, x, res)
-    p_box, a_box = run(box, x[:nb], res[:nb])
-    p_sp, a_sp = run(sparse, x[nb:], res[nb:])
-    assert np.array_equal(p_all[:nb], p_box) and np.array_equal(p_all[nb:], p_sp)
-    assert np.array_equal(a_all[:nb], a_box) and np.array_equal(a_all[nb:], a_sp)
     rows = sample_rows(n, 300)
     exp = orc.Rulebook(both).conv(x, w, bias, ci, co, rows=rows)
-    err = max_rel_err(p_all[rows[0]:rows[1]:rows[2]], exp)
     e_add = sh.storage_round(orc.add(sh.storage_round(exp, dtype), res[rows[0]:rows[1]:rows[2]]), dtype)
-    err_add = max_rel_err(a_all[rows[0]:rows[1]:rows[2]], e_add)
-    say(f"conv layouts ci={ci} co={co} max_rel_err={err:.3e} add={err_add:.3e}")
-    assert err <= TOL[dtype] and err_add <= TOL[dtype]
+    for be in schedules[dtype]:
+        p_all, a_all = run(be, both, x, res)
+        p_box, a_box = run(be, box, x[:nb], res[:nb])
+        p_sp, a_sp = run(be, sparse, x[nb:], res[nb:])
+        assert np.array_equal(p_all[:nb], p_box) and np.array_equal(p_all[nb:], p_sp)
+        assert np.array_equal(a_all[:nb], a_box) and np.array_equal(a_all[nb:], a_sp)
+        err = max_rel_err(p_all[rows[0]:rows[1]:rows[2]], exp)
+        err_add = max_rel_err(a_all[rows[0]:rows[1]:rows[2]], e_add)
+        say(f"conv layouts ci={ci} co={co} max_rel_err={err:.3e} add={err_add:.3e}")
+        assert err <= TOL[dtype] and err_add <= TOL[dtype]
 
 
 @pytest.mark.parametrize("dtype", [sh.BF16, sh.F16])
 @pytest.mark.parametrize("n", [1, 2, 127, 129, 257])
 @pytest.mark.parametrize("ci,co", [(256, 512), (128, 256), (512, 256)])
-def test_conv_wide_outputs_tiny_sets(backends, dtype, n, ci, co):
+def test_conv_wide_outputs_tiny_sets(schedules, dtype, n, ci, co):
     """Co % 256 == 0 on sets of one to two map tiles (a single voxel, a short
     second half tile, one row past a tile), with the plain and the in-place
     residual epilogue, against the oracle on every row."""
-    be = backends[dtype]
     g = np.stack(np.meshgrid(*(np.arange(7),) * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
     coords = np.ascontiguousarray(np.concatenate([np.zeros((n, 1), np.int64), g], 1).astype(np.int32))
     rng = np.random.default_rng(n * 3 + ci + co + dtype)
@@ -266,16 +279,17 @@ def test_conv_wide_outputs_tiny_sets(backends, dtype, n, ci, co):
     w = sh.storage_round(rng.standard_normal((co, 27, ci)) / math.sqrt(27 * ci), dtype)
     bias = (0.1 * rng.standard_normal(co)).astype(np.float32)
     res = sh.storage_round(rng.standard_normal((n, co)), dtype)
-    rb = be.build_rulebook(coords)
-    xb, yb = be.upload(x), be.alloc(n * co)
-    be.conv(rb, xb, w, bias, yb, ci, co)
     exp = orc.Rulebook(coords).conv(x, w, bias, ci, co)
-    assert max_rel_err(be.download(yb).reshape(n, co), exp) <= TOL[dtype]
-    r = be.upload(res)
-    be.conv_add(rb, xb, w, bias, r, r, ci, co)
     e_add = sh.storage_round(orc.add(sh.storage_round(exp, dtype), res), dtype)
-    assert max_rel_err(be.download(r).reshape(n, co), e_add) <= TOL[dtype]
-    rb.free()
+    for be in schedules[dtype]:
+        rb = be.build_rulebook(coords)
+        xb, yb = be.upload(x), be.alloc(n * co)
+        be.conv(rb, xb, w, bias, yb, ci, co)
+        assert max_rel_err(be.download(yb).reshape(n, co), exp) <= TOL[dtype]
+        r = be.upload(res)
+        be.conv_add(rb, xb, w, bias, r, r, ci, co)
+        assert max_rel_err(be.download(r).reshape(n, co), e_add) <= TOL[dtype]
+        rb.free()
 
 
 def decoder_level_set(levels):
@@ -294,11 +308,10 @@ def decoder_level_set(levels):
 
 
 @pytest.mark.parametrize("levels,ci,co", [(1, 512, 512), (1, 512, 2048), (2, 256, 256), (2, 256, 1024), (3, 128, 512)])
-def test_conv_decoder_levels_vs_oracle(backends, levels, ci, co):
+def test_conv_decoder_levels_vs_oracle(schedules, levels, ci, co):
     """The decoder's sparse levels at their real size and widths (the
     ConvNeXt convs and the up-blocks' Ci -> 8 Co convs), bf16, against the
     oracle on a strided sample that puts a row in every 256-row map tile."""
-    be = backends[sh.BF16]
     coords = decoder_level_set(levels)
     n = coords.shape[0]
     rng = np.random.default_rng(levels * 1000 + ci + co)
@@ -306,16 +319,17 @@ def test_conv_decoder_levels_vs_oracle(backends, levels, ci, co):
     w = sh.storage_round(rng.standard_normal((co, 27, ci)) / math.sqrt(27 * ci), sh.BF16)
     bias = (0.1 * rng.standard_normal(co)).astype(np.float32)
     say(f"decoder level {levels} conv {ci}->{co} n={n}")
-    rb = be.build_rulebook(coords)
-    xb, yb = be.upload(x), be.alloc(n * co)
-    be.conv(rb, xb, w, bias, yb, ci, co)
-    got = be.download(yb).reshape(n, co)
     rows = (5, n, 255)
     exp = orc.Rulebook(coords).conv(x, w, bias, ci, co, rows=rows)
-    err = max_rel_err(got[rows[0]:rows[1]:rows[2]], exp)
-    say(f"decoder level {levels} conv {ci}->{co} rows={exp.shape[0]} max_rel_err={err:.3e}")
-    assert err <= TOL[sh.BF16]
-    rb.free()
+    for be in schedules[sh.BF16]:
+        rb = be.build_rulebook(coords)
+        xb, yb = be.upload(x), be.alloc(n * co)
+        be.conv(rb, xb, w, bias, yb, ci, co)
+        got = be.download(yb).reshape(n, co)
+        err = max_rel_err(got[rows[0]:rows[1]:rows[2]], exp)
+        say(f"decoder level {levels} conv {ci}->{co} rows={exp.shape[0]} max_rel_err={err:.3e}")
+        assert err <= TOL[sh.BF16]
+        rb.free()
 
 
 _ENCODER_SETS = {}
@@ -337,11 +351,10 @@ def encoder_level_set(level):
 
 @pytest.mark.parametrize("level,ci,co", [(0, 64, 16), (1, 128, 32), (2, 256, 256), (3, 512, 512), (3, 512, 128),
                                          (4, 1024, 1024)])
-def test_conv_encoder_levels_vs_oracle(backends, level, ci, co):
+def test_conv_encoder_levels_vs_oracle(schedules, level, ci, co):
     """The encoder's levels at their real size and widths (the ConvNeXt convs
     and the down-blocks' Ci -> Co / 8 convs), bf16, against the oracle on a
     strided sample that puts a row in every 256-row map tile."""
-    be = backends[sh.BF16]
     coords = encoder_level_set(level)
     n = coords.shape[0]
     rng = np.random.default_rng(level * 1000 + ci + co)
@@ -349,16 +362,17 @@ def test_conv_encoder_levels_vs_oracle(backends, level, ci, co):
     w = sh.storage_round(rng.standard_normal((co, 27, ci)) / math.sqrt(27 * ci), sh.BF16)
     bias = (0.1 * rng.standard_normal(co)).astype(np.float32)
     say(f"encoder level {level} conv {ci}->{co} n={n}")
-    rb = be.build_rulebook(coords)
-    xb, yb = be.upload(x), be.alloc(n * co)
-    be.conv(rb, xb, w, bias, yb, ci, co)
-    got = be.download(yb).reshape(n, co)
     rows = (7, n, 255)
     exp = orc.Rulebook(coords).conv(x, w, bias, ci, co, rows=rows)
-    err = max_rel_err(got[rows[0]:rows[1]:rows[2]], exp)
-    say(f"encoder level {level} conv {ci}->{co} rows={exp.shape[0]} max_rel_err={err:.3e}")
-    assert err <= TOL[sh.BF16]
-    rb.free()
+    for be in schedules[sh.BF16]:
+        rb = be.build_rulebook(coords)
+        xb, yb = be.upload(x), be.alloc(n * co)
+        be.conv(rb, xb, w, bias, yb, ci, co)
+        got = be.download(yb).reshape(n, co)
+        err = max_rel_err(got[rows[0]:rows[1]:rows[2]], exp)
+        say(f"encoder level {level} conv {ci}->{co} rows={exp.shape[0]} max_rel_err={err:.3e}")
+        assert err <= TOL[sh.BF16]
+        rb.free()
 
 
 @pytest.mark.parametrize("ci,co,n", [(512, 128, 2100), (384, 64, 1500)])

@@ -1,6 +1,7 @@
 """The 16-bit COMPACT policy, whose kernel map is built as pair lists: both forms of the map against the oracle, whichever
 is asked for first; convs on a built map when no memory is left (a compacted conv needs none; 64 -> 64, which takes the
-row table where it fits, then walks the lists); and the mesh extraction, which reads the row table.
+row table where it fits, then walks the lists); the mesh extraction, which reads the row table; and features past the
+2 GiB that AUTO's kernels address.
 
 Tolerance where two schedules are compared: they differ by the order of their fp32 sums and one unit in the last place of
 the storage type where those fall on either side of a tie (2^-7 of the value in bf16, 2^-10 in fp16; 1e-4 for the sums)."""
@@ -90,3 +91,32 @@ def test_mesh():
         be.destroy()
     assert mesh[0][1].shape[0] > 0
     assert np.array_equal(mesh[0][0], mesh[1][0]) and np.array_equal(mesh[0][1], mesh[1][1])
+
+
+def test_features_past_2_gib():
+    """524,300 rows of 2,048 fp16 channels are more than the sorted conv's and the GEMM's loads address: the conv takes the
+    compacted kernel, the linear the MFMA linear kernel.  Rows repeat a block of 1,000, and sampled outputs, among them
+    rows whose sources lie past 2 GiB, are compared with 64-bit sums over their neighbours."""
+    dtype, ci, co, n = sh.F16, 2048, 16, 524300
+    rng = np.random.default_rng(1)
+    c = np.ascontiguousarray(wl.make_coords(4)[:n])
+    block = sh.storage_round(rng.standard_normal((1000, ci)), dtype)
+    raw = np.concatenate([np.tile(block.astype(np.float16), (n // 1000, 1)), block[:n % 1000].astype(np.float16)])
+    w = sh.storage_round(rng.standard_normal((co, 27, ci)) / math.sqrt(27 * ci), dtype)
+    lw = sh.storage_round(rng.standard_normal((128, ci)) / math.sqrt(ci), dtype)
+    be = sh.Backend(0, dtype, linear_algo=sh.LINEAR_KERNEL)
+    xb, yb, zb = be.upload_raw(raw.view(np.uint16)), be.alloc(n * co), be.alloc(n * 128)
+    rb = be.build_rulebook(c)
+    be.conv(rb, xb, w, None, yb, ci, co)
+    be.linear(xb, lw, None, zb, n, ci, 128)
+    y, z = be.download(yb).reshape(n, co), be.download(zb).reshape(n, 128)
+    rb.free()
+    be.destroy()
+    rows = np.unique(np.concatenate([np.arange(0, n, 3001), np.arange(n - 64, n)]))
+    nbr = orc.Rulebook(c).neighbors()[rows]
+    exp = np.zeros((rows.size, co))
+    for k in range(27):
+        has = nbr[:, k] >= 0
+        exp[has] += block[nbr[has, k] % 1000].astype(np.float64) @ w[:, k].T.astype(np.float64)
+    for got, want in ((y[rows], exp), (z[rows], block[rows % 1000].astype(np.float64) @ lw.T.astype(np.float64))):
+        assert np.max(np.abs(got - want) / np.maximum(1.0, np.abs(want))) <= TOL[dtype]

@@ -174,6 +174,33 @@ def test_more_rows_than_a_sort_window(backends):
     assert err(y[::1009], sh.storage_round(exp, dtype)) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("c", [128, 256, 512])
+def test_block_repeats_bit_for_bit(backends, c):
+    """A whole ConvNeXt block on rulebooks built anew, in row order and in mask order, whose ties among rows of one bucket
+    fall as the atomics do: the same bits each time."""
+    dtype = sh.BF16
+    be = backends[dtype]
+    rng = np.random.default_rng(c)
+    coords = np.ascontiguousarray(wl.make_coords(2)[:30000])
+    n = coords.shape[0]
+    x = be.upload(rng.standard_normal((n, c), dtype=np.float32))
+    w, w0, w2 = (be.keep(np.ascontiguousarray(a, np.float32)) for a in
+                 (weights(rng, c, c, dtype), rng.standard_normal((4 * c, c)) / math.sqrt(c),
+                  rng.standard_normal((c, 4 * c)) / math.sqrt(4 * c)))
+    got = []
+    for _ in range(3):
+        rb = be.build_rulebook(coords)
+        for ordered in (False, True):
+            if ordered:
+                reach_order(be, rb)
+            y = be.alloc(n * c)
+            be.convnext_block(rb, x, w, None, None, None, w0, None, w2, None, y, c, 1e-6)
+            got.append(be.download_raw(y))
+        rb.free()
+    for g in got[1:]:
+        assert np.array_equal(g, got[0])
+
+
 @pytest.mark.parametrize("algo", [sh.CONV_AUTO, sh.CONV_MASKED, sh.CONV_COMPACT])
 @pytest.mark.parametrize("ci,co", [(64, 64), (128, 128), (192, 64), (320, 16), (96, 128)])
 @pytest.mark.parametrize("bad", [np.inf, np.nan])

@@ -3,8 +3,8 @@
 Each case draws a voxel set (uniform box, Gaussian clusters or repeated
 rows, up to 6,000 voxels), channel counts, storage type, conv policy and
 epilogue, so that every dispatch branch of the backend's conv runs on
-irregular sets: the output-stationary 64 -> 64 kernel, 256-channel blocks over
-half tiles, 4- and 8-wavefront 128-channel blocks, 64/32/16-channel blocks,
+irregular sets: the sorted kernel (AUTO), the compacted 256-channel blocks over
+half tiles, 4- and 8-wavefront 128-channel blocks and 64/32/16-channel blocks,
 the masked schedule and the VALU kernel for shapes MFMA does not take.  The
 oracle (trellis_sparse_cpu.c:324-373 restated) computes a strided sample of
 output rows from the same rounded inputs; the bar is the storage tolerance of
