@@ -782,7 +782,7 @@ def run_block(args):
 def conv_schedule(dtype, ci, co, algo):
     """Name of the conv kernel the backend runs (its fallback rules)."""
     mfma = dtype != sh.F32 and ci % 32 == 0 and co % 64 == 0
-    if algo == sh.CONV_AUTO and mfma and ci % 64 == 0:
+    if mfma and ci % 64 == 0 and (algo == sh.CONV_AUTO or (algo == sh.CONV_COMPACT and ci == 64 and co == 64)):
         return "sorted"  # output-stationary kernel over rows in mask order
     if algo == sh.CONV_COMPACT and mfma and co % 256 == 0 and ci % 128 == 0:
         return "compact256"  # 256-channel blocks over half map tiles
@@ -952,16 +952,20 @@ def main():
     per_launch_flops = wl.conv_flops(job.pairs, job.ci, job.co)
     achieved = per_launch_flops / (conv_avg * 1e-3) / 1e12 if conv_avg > 0 else 0.0
     hm_ms = (stages["hash"][0] + stages["map"][0]) / args.steps
-    # Hash + kernel map against HBM: the work definition's bytes (hash 28 N,
-    # map 16 N + 108 N + 8 P + 216, the 108 N being an [N][27] neighbour
-    # table), and the bytes the production build moves (hash 28 N; map 16 N
-    # coordinates + 112 N rows of 27 neighbours and the mask + 4 N masks; where
-    # the conv takes the rows in mask order also 16 N: masks twice, 2-byte ranks
-    # out and in, places).
+    # Hash + kernel map against HBM.  Needed bytes: what the build reads and
+    # leaves, once each (hash 28 N; map 16 N coordinates, 112 N rows of 27
+    # neighbours and the mask, 4 N masks; the mask order's 4 N places, where the
+    # conv takes the rows in it).  Moved bytes: the order's passes too (masks
+    # read twice, 2-byte ranks out and in, and per 4,096 rows 64 KB of bucket
+    # counts written, read and written back, of which each row reads 8 bytes).
+    # Definition bytes: a dense [N][27] neighbour table and 8 bytes per pair of
+    # lists (28 N + 16 N + 108 N + 8 P + 216), which this build does not write.
     hm_def_bytes = wl.hash_bytes(job.m) + wl.map_bytes(job.m, job.pairs)
     algo_name = conv_schedule(spec["dtype"], job.ci, job.co, args.conv_algo)
-    hm_moved_bytes = (28.0 + 16.0 + 112.0 + 4.0 + (16.0 if algo_name == "sorted" else 0.0)) * job.m
-    hm_gbs = hm_def_bytes / (hm_ms * 1e-3) / 1e9 if hm_ms > 0 else 0.0
+    ordered = algo_name == "sorted"
+    hm_needed_bytes = (28.0 + 16.0 + 112.0 + 4.0 + (4.0 if ordered else 0.0)) * job.m
+    hm_moved_bytes = hm_needed_bytes + (20.0 * job.m + 3.0 * 65536.0 * ((job.m + 4095) // 4096) if ordered else 0.0)
+    hm_gbs = hm_needed_bytes / (hm_ms * 1e-3) / 1e9 if hm_ms > 0 else 0.0
     elem = 4 if spec["dtype"] == sh.F32 else 2
     # The conv's binding roofline: compute (2 P Ci Co at the dtype's MFMA or
     # fp32 peak) or HBM (compulsory bytes at 8 TB/s), whichever takes longer.
@@ -1001,7 +1005,7 @@ def main():
         "hash_map_roofline": {
             "bound": "hbm", "achieved": round(hm_gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
             "frac": round(hm_gbs / PEAK_HBM_GBS, 4), "ms_per_step": round(hm_ms, 4),
-            "definition_bytes": hm_def_bytes, "moved_bytes": hm_moved_bytes,
+            "needed_bytes": hm_needed_bytes, "definition_bytes": hm_def_bytes, "moved_bytes": hm_moved_bytes,
             "moved_gbs": round(hm_moved_bytes / (hm_ms * 1e-3) / 1e9, 1) if hm_ms > 0 else 0.0,
         },
         "conv_kernel_tflops": round(achieved, 2),

@@ -107,7 +107,7 @@ struct Backend {
     // and the event the host spins on for them (allocated at creation).
     int32_t * host_words = nullptr;
     hipEvent_t words_ready = nullptr;
-    // Stream and event for a download that overlaps the backend stream's later
+    // Stream and event for a download queued beside the backend stream's later
     // work (the mesh vertices; created on first use).
     hipStream_t copy_stream = nullptr;
     hipEvent_t copy_from = nullptr;
@@ -796,10 +796,10 @@ trellis_status mlp_impl(trellis_sparse_backend * backend, const trellis_sparse_b
     }
     // C = 256 on few rows: the fused kernel's 128-row blocks leave most CUs
     // idle and each still walks the whole hidden layer (0.040 ms from 1,000 to
-    // 10,000 rows); composed on the GEMM kernel, with the same roundings, 0.021
-    // ms on 1,000 rows, 0.028 on 5,003, 0.036 on 10,000, 0.054 (fused 0.046)
-    // on 20,000.  The fused kernel needs no intermediates and takes over where
-    // they do not fit; row_norm refuses eps = 0.
+    // 10,000 rows on 256 CUs); composed on the GEMM kernel, with the same
+    // roundings, 0.021 ms on 1,000 rows, 0.028 on 5,003, 0.036 on 10,000, 0.054
+    // (fused 0.046) on 20,000.  The fused kernel needs no intermediates and
+    // takes over where they do not fit; row_norm refuses eps = 0.
     constexpr int64_t kComposed256Rows = 12000;
     if (c == 256 && n <= kComposed256Rows && eps > 0.0f) {
         const trellis_status st =
@@ -1072,8 +1072,9 @@ trellis_status op_build_rulebook(trellis_sparse_backend * backend, const int32_t
 }
 
 // The conv, optionally with a fused epilogue (fused_epi != nullptr: row
-// norm (+ SiLU) or residual add, compacted schedule only).  epi's gamma and
-// beta are host pointers here; they go through the weight cache.
+// norm (+ SiLU) or residual add; the sorted and compacted schedules have them,
+// at the compacted one's widths, so that either can run).  epi's gamma and beta
+// are host pointers here; they go through the weight cache.
 trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_rulebook * rulebook,
                          const trellis_sparse_buffer * feats, const float * weight, const float * bias,
                          trellis_sparse_buffer * out, int64_t n, int ci, int co, const ConvEpilogue * fused_epi,
@@ -1093,7 +1094,8 @@ trellis_status conv_impl(trellis_sparse_backend * backend, const trellis_sparse_
         const bool shape_ok = fused_epi->mode == kEpiNorm ? co == 128 : co % 128 == 0;
         if (!algo_ok || !conv_stream_supported(dt, ci, co) || !shape_ok) {
             const std::string msg = std::string(what) +
-                                    ": needs the compacted conv (16-bit, Ci 64 or a multiple of 128) and " +
+                                    ": needs the AUTO or COMPACT conv policy, 16-bit storage, Ci 64 or a multiple of "
+                                    "128 and " +
                                     (fused_epi->mode == kEpiNorm ? "Co == 128" : "Co a multiple of 128");
             return fail(be, TRELLIS_STATUS_NOT_IMPLEMENTED, msg.c_str());
         }
@@ -1832,9 +1834,11 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
         }
         st = hip_status(be, err, "flex_dual_grid_mesh copy stream");
     }
-    // Check and vertices first: the vertices travel to pinned memory on the
-    // copy stream while the backend stream builds the corner map and counts
-    // the quads.
+    // Check and vertices first: the vertices go to pinned memory on the copy
+    // stream, and the map's launches need not wait for the host to see them
+    // arrive.  (The transfer and the map hardly overlap on the device: the
+    // hash's clear, started beside the transfer, ends with it, 135 us instead
+    // of 10 at 1,263,630 voxels, and the map follows.)
     bool copying = false;
     if (st == TRELLIS_STATUS_OK) {
         stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);

@@ -1347,7 +1347,7 @@ hipError_t launch_conv_generic(int dtype, const void * x, const int32_t * nbr, c
     // rows 0.013 against 0.010 and 0.081 against 0.054).
     if (dtype == kF32 && n > 1 && ci % 32 == 0 && co % 4 == 0 && 108ll * ci * co <= (int64_t) INT32_MAX) {
         // Rows per wavefront: more of them share a wavefront's weight reads,
-        // fewer give the GPU more wavefronts.  Measured (ms, R = 1 / 2 / 4 /
+        // fewer give the GPU (256 CUs) more wavefronts.  Measured (ms, R = 1 / 2 / 4 /
         // 8, k_conv_generic last): 1,500 rows 64 -> 64 0.026 / 0.035 / 0.055 /
         // 0.094, 0.096; 5,000 rows 32 -> 64 0.023 / 0.026 / 0.032 / 0.054,
         // 0.055; 14,648 rows 64 -> 64 (config 1) 0.111 / 0.100 / 0.088 /

@@ -12,8 +12,11 @@ namespace {
 // implicit GEMM over (offset with a neighbour in the block, input channel).
 // Rows with like masks share blocks, so 0.65-0.93 of the row-offsets a block
 // multiplies have a neighbour on voxelised surfaces (0.55 where the children
-// of a subdivision are random), which costs less than compacting the valid
-// pairs: no unit lists, no tile sums in LDS, no scatter.
+// of a subdivision are random; the choice of a shape below does not look at
+// it), which costs less than compacting the valid pairs: no unit lists, no tile
+// sums in LDS, no scatter.  Not so on voxels scattered at random in few
+// channels (300,000 at 20 %: 64 -> 16 54 us, compacted 54, 128 -> 32 100 and
+// 92; from 128 -> 128 on it is the faster one).
 //
 // RW x CW wavefronts hold BM / RW rows x BN / CW channels each.  Each K step
 // (32 input channels of one offset) brings BM gathered rows' 64 bytes and
@@ -41,7 +44,7 @@ namespace {
 // Measured against the compacted schedule (ms, conv alone): 128 -> 128 on
 // 419,341 rows 0.60 -> 0.31; 256 -> 1024 on 350,000 5.1 -> 2.7; 512 -> 512 on
 // 79,523 1.11 -> 0.71; 1024 -> 1024 on 18,216 1.12 -> 0.77; 256 -> 256 on
-// 5,003 0.100 -> 0.035; 64 -> 64 on 3,788,747 1.11 -> 0.85; 256 -> 128 on
+// 5,003 0.100 -> 0.036; 64 -> 64 on 3,788,747 1.11 -> 0.85; 256 -> 128 on
 // 1,259,866 random children 1.71 -> 1.56.
 template <int DT, int BM, int BN, int RW, int CW, int SLOTS, bool PP = false>
 __global__ void __launch_bounds__(64 * RW * CW, RW * CW == 8 ? 2 : 1)
@@ -318,7 +321,8 @@ constexpr Shape kShapes[] = {
 // The shape that finishes first: large blocks do the most MFMA work per
 // fetched byte (256 -> 1024 on 350,000 rows: 2.77 ms with 256 x 256, 3.11 with
 // 128 x 256), small ones fill the GPU on small sets (256 -> 256 on 5,003 rows:
-// 0.113 ms with 256 x 256, 0.076 with 128 x 256, 0.035 with 64 x 64), and
+// 0.113 ms with 256 x 256, 0.074 with 128 x 256, 0.061 with 96 x 256, 0.049
+// with 128 x 128, 0.036 with 64 x 128, which is taken, 0.033 with 64 x 64), and
 // between these the row count decides which fills its last round (1024 -> 1024
 // on 18,216 rows: 0.93, 0.85, 0.81, 0.77 and 0.86 ms down the list; 256 -> 256
 // on 80,000: 0.253, 0.234, 0.205, 0.193 and 0.213; on 20,000: 0.122, 0.116,

@@ -234,7 +234,7 @@ hipError_t launch_conv_generic(int dtype, const void * x, const int32_t * nbr, c
 bool conv_mfma_supported(int dtype, int ci, int co);
 hipError_t launch_conv_mfma_masked(int dtype, const void * x, const int32_t * rows, const void * w16,
                                    const float * bias, void * y, int64_t n, int ci, int co, hipStream_t s);
-// Epilogue of the 128-channel compacted conv: after bias and the rounding to
+// Epilogue of the sorted and the compacted conv: after bias and the rounding to
 // the storage type, optionally a row norm (+ SiLU) over whole rows (co ==
 // 128, one block holds every channel of its rows) or a residual add
 // (rounded again), as the slot sequences conv -> row_norm(_silu) and
