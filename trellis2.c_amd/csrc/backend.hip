@@ -1834,11 +1834,12 @@ trellis_status fdg_mesh_impl(trellis_sparse_backend * backend, const int32_t * c
         }
         st = hip_status(be, err, "flex_dual_grid_mesh copy stream");
     }
-    // Check and vertices first: the vertices go to pinned memory on the copy
-    // stream, and the map's launches need not wait for the host to see them
-    // arrive.  (The transfer and the map hardly overlap on the device: the
-    // hash's clear, started beside the transfer, ends with it, 135 us instead
-    // of 10 at 1,263,630 voxels, and the map follows.)
+    // Check and vertices first: the vertices travel to pinned memory on the
+    // copy stream while the backend stream builds the corner map and counts
+    // the quads.  (So it is where the runtime moves them with a copy engine.
+    // Where it copies with a kernel, as seen in processes that also load torch,
+    // the hash's clear beside it ends with it, 135 us instead of 10 at 1,263,630
+    // voxels, and the map only follows.)
     bool copying = false;
     if (st == TRELLIS_STATUS_OK) {
         stage_begin(be, TRELLIS_SPARSE_HIP_STAGE_ELEMENTWISE);
