@@ -183,9 +183,10 @@ typedef enum trellis_sparse_hip_dtype {
 } trellis_sparse_hip_dtype;
 
 /* Convolution schedule.  AUTO picks by channel counts and dtype: for F16/BF16
- * with Ci % 64 == 0 and Co 16, 32 or a multiple of 64 an MFMA kernel over rows
- * in the order of their neighbour masks (finite weights, features up to 2
- * GiB), else COMPACT where it applies, else MASKED, else GENERIC; a schedule
+ * with Ci % 64 == 0 and Co 16, 32 or a multiple of 64 an MFMA kernel that takes
+ * the rows in the order of their neighbour masks once the convs on a rulebook
+ * pay for sorting them (finite weights, features up to 2 GiB), else COMPACT
+ * where it applies, else MASKED, else GENERIC; a schedule
  * that does not apply falls back the same way, and so does MASKED (to GENERIC)
  * for weights with an infinity or NaN, which it would multiply with the zeros
  * of missing neighbours.  The choice never changes which pairs contribute, only
@@ -195,7 +196,8 @@ typedef enum trellis_sparse_hip_conv_algo {
     TRELLIS_SPARSE_HIP_CONV_GENERIC = 1,   /* one lane per output element, any channels and dtype */
     TRELLIS_SPARSE_HIP_CONV_MASKED = 2,    /* MFMA over the neighbour table; F16/BF16, Ci % 32 == 0, Co % 64 == 0 */
     TRELLIS_SPARSE_HIP_CONV_COMPACT = 3    /* MFMA over compacted per-tile pair lists; F16/BF16, Ci == 64 or
-                                              Ci % 128 == 0, Co % 64 == 0 */
+                                              Ci % 128 == 0, Co 16, 32 or a multiple of 64 (64 -> 64 runs AUTO's
+                                              kernel) */
 } trellis_sparse_hip_conv_algo;
 
 /* Which code runs the linear and linear_silu slots in 16-bit storage. */
