@@ -91,6 +91,7 @@ def test_convnext_tail_256_vs_oracle(backends, n):
         finally:
             be.fail_alloc(-1)
         got = be.download(yb).reshape(n, c)[rows]
+        assert sh.LIB.trellis_sparse_hip_last_error(be.ptr) == b""
         assert np.max(np.abs(got - e) / np.maximum(1.0, np.abs(e))) <= tol
 
     check(1e-6)

@@ -751,11 +751,11 @@ trellis_status norm_impl(trellis_sparse_backend * backend, const trellis_sparse_
                          const float * beta, trellis_sparse_buffer * y, int64_t n, int c, float eps, int silu);
 
 // The tail at c >= 512 (a multiple of 128), where a tile's normalised rows
-// would fill the LDS: row_norm into an n x c intermediate, mlp0 + SiLU into
-// an n x 4c intermediate, and mlp2 with the residual added to its fp32 sums
-// (GEMM library epilogue; the kernels' fallback adds the rounded mlp2 output
-// as the slot sequence does).  The n x c intermediate is mlp2's scratch for
-// that fallback.
+// would fill the LDS, and at c = 256 on few rows: row_norm into an n x c
+// intermediate, mlp0 + SiLU into an n x 4c intermediate, and mlp2 with the
+// residual added to its fp32 sums (GEMM library epilogue) or to its rounded
+// output as the slot sequence does (the kernels; the GEMM kernel in its
+// epilogue, the others through the n x c intermediate as scratch).
 bool mlp_composed_supported(int dtype, int c) { return (dtype == kF16 || dtype == kBF16) && c >= 512 && c % 128 == 0; }
 
 trellis_status mlp_composed(trellis_sparse_backend * backend, const trellis_sparse_buffer * x, const float * gamma,
@@ -805,6 +805,7 @@ trellis_status mlp_impl(trellis_sparse_backend * backend, const trellis_sparse_b
         const trellis_status st =
             mlp_composed(backend, x, gamma, beta, w0, b0, w2, b2, residual, y, n, c, eps, false);
         if (st != TRELLIS_STATUS_OUT_OF_MEMORY) return st;
+        be->last_error.clear();
     }
     CallScope scope(be);
     const void *g = nullptr, *bt = nullptr, *pw0 = nullptr, *pb0 = nullptr, *pw2 = nullptr, *pb2 = nullptr;
